@@ -185,11 +185,13 @@ int pf_pcg(pf_ctx* ctx, int op, const double* b_free, double* x_free, double eps
 /* Form of the Jacobi-PCG recurrences for the quad4 matrix-free solves of
  * this context (pf_pcg and pf_pcg_dev with PF_OP_EBE64 / PF_OP_EBE32, and
  * pf_simp_run), until changed.  PF_PCG_SCALINGCG (the default) is
- * ScalingCG's own order (CG.h:419-453), two launches per iteration.  The
+ * ScalingCG's own order (CG.h:419-453), two reductions per iteration.  The
  * single-reduction forms follow Chronopoulos and Gear (p.Kp from u.Ku): one
- * launch and one reduction per iteration, the same iterates in exact
- * arithmetic, the same stopping test on the recursive residual, the Jacobi
- * step as a product with 1/D.
+ * reduction per iteration, the same iterates in exact arithmetic, the same
+ * stopping test on the recursive residual, the Jacobi step as a product with
+ * 1/D.  Grids whose vectors fit the registers and LDS of the chip (up to
+ * about 650,000 nodes) are solved by one resident kernel in the first three
+ * forms; larger ones, and the recomputed form, launch every iteration:
  *   PF_PCG_SINGLE_REDUCTION_CARRIED: s = K p and w = K u carried as vectors
  *     (88 bytes per free DOF and iteration);
  *   PF_PCG_SINGLE_REDUCTION_RECOMPUTED: s = K p recomputed from p on a

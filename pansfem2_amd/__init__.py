@@ -344,7 +344,7 @@ class Context:
 
     def set_pcg_form(self, form):
         """PF_PCG_SCALINGCG (ScalingCG's order, the default) or a
-        single-reduction form (one launch per iteration) for the FP64 quad4
+        single-reduction form (one reduction per iteration) for the FP64 quad4
         matrix-free solves of this context: PF_PCG_SINGLE_REDUCTION_CARRIED
         (s = K p carried), PF_PCG_SINGLE_REDUCTION_RECOMPUTED (s = K p
         recomputed on a two-node halo) or PF_PCG_SINGLE_REDUCTION (the

@@ -2,6 +2,7 @@
 // filter, OC and the device-resident SIMP loop.  Declarations and the
 // reference routine each entry point replaces: include/pansfem2_amd.h.
 #include "pf_kernels.hip"
+#include "pf_resident.hip"
 #include "pf_mma.hip"
 #include "pf_hex8.hip"
 #include "pf_learned.hip"
@@ -253,6 +254,7 @@ void free_grid(pf_ctx* ctx) {
     dfree(ctx->f_x); dfree(ctx->f_r); dfree(ctx->f_z); dfree(ctx->f_q); dfree(ctx->f_p0); dfree(ctx->f_p1);
     dfree(ctx->d_s0); dfree(ctx->d_s1); dfree(ctx->f_s0); dfree(ctx->f_s1); dfree(ctx->d_Dinv);
     dfree(ctx->f_D); dfree(ctx->f_b);
+    dfree(ctx->res_halo);
     dfree(ctx->d_e0); dfree(ctx->d_e1); dfree(ctx->d_e2); dfree(ctx->d_e3); dfree(ctx->d_e4); dfree(ctx->d_e5);
     dfree(ctx->d_e6);
     dfree(ctx->d_cg); dfree(ctx->d_load);
@@ -409,6 +411,139 @@ struct EventPair {
     }
 };
 
+// ------------------------------------------------- resident solves -----
+// Tiles of a resident solve: gi x gj workgroups of nt threads, S node rows
+// per thread.  gi == 0: the grid does not fit.
+struct ResShape {
+    int gi = 0, gj = 0, nt = 0, S = 0;
+    size_t lds = 0;
+};
+constexpr size_t kResLds = 150 * 1024;  // of a CU's 160 KB, beside the static part
+constexpr int kResConfigs[][2] = {{256, 1}, {256, 2}, {512, 2}, {512, 4}, {512, 5}};
+
+// The tiling with the least estimated time per iteration, in microseconds over
+// what every tiling pays: 0.0012 per node (with the rows that pad a tile to S),
+// up to half as much again where a wave spans several short tile rows (LDS
+// conflicts: 1024x512 as 16x16 tiles of 65x33 nodes 7.2, as 32x8 of 33x65
+// 6.1), 0.003 per halo node pair, 0.4 for the longer pause of more than 64
+// workgroups (res_pause), and 1.2 less for a single one, which waits for nobody (31x15:
+// 2.0 against 3.1).
+template <class T>
+ResShape res_pick(const pf_ctx* ctx) {
+    ResShape best;
+    double bestc = 0.0;
+    const int ni = ctx->nx + 1, nj = ctx->ny + 1;
+    for (const auto& cfg : kResConfigs) {
+        const int nt = cfg[0], S = cfg[1];
+        for (int gi = 1; gi <= std::min(ni, ctx->res_wgs); gi++)
+            for (int gj = 1; gj <= std::min(nj, ctx->res_wgs / gi); gj++) {
+                const int ti = (ni + gi - 1) / gi, tj = (nj + gj - 1) / gj;
+                const int rows = (ti + S - 1) / S * S;
+                const size_t lds = res_lds_bytes<T>(ti, tj, S, nt);
+                if (rows / S * tj > nt || 2 * (tj + 2) + 2 * ti > nt || lds > kResLds) continue;
+                const double split = std::min(1.0, std::max(0.0, 64.0 / tj - 1.0));
+                const double cost = 0.0012 * rows * tj * (1.0 + 0.5 * split) + 0.003 * (ti + tj) + 0.0002 * S * nt +
+                                    (gi * gj == 1 ? -1.2 : gi * gj > 64 ? 0.4 : 0.0);
+                if (best.gi == 0 || cost < bestc) {
+                    bestc = cost;
+                    best.gi = gi;
+                    best.gj = gj;
+                    best.nt = nt;
+                    best.S = S;
+                    best.lds = lds;
+                }
+            }
+    }
+    return best;
+}
+
+template <class T, bool SR>
+const void* res_kernel(const ResShape& sh) {
+#define PF_RES_CASE(NT_, S_) \
+    if (sh.nt == NT_ && sh.S == S_) return (const void*)k_pcg_q4_resident<T, S_, NT_, SR>;
+    PF_RES_CASE(256, 1)
+    PF_RES_CASE(256, 2)
+    PF_RES_CASE(512, 2)
+    PF_RES_CASE(512, 4)
+    PF_RES_CASE(512, 5)
+#undef PF_RES_CASE
+    return nullptr;
+}
+
+// Jacobi-PCG resident on the chip (k_pcg_q4_resident); *ran is false, and
+// nothing has been solved, when the grid does not fit or the launch cannot be
+// made or stalled: the caller then launches per iteration.  D: the diagonal,
+// or its inverse for the single-reduction form (sr).
+constexpr int kResChunk = 2048;  // iterations per launch: other streams get the GPU in between
+template <class T>
+int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s, T* p, T* w, double eps, int itrmax,
+                 PcgRun& out, bool* ran) {
+    *ran = false;
+    if (ctx->res_wgs < 1 || ctx->res_stalled) return PF_OK;
+    const ResShape sh = res_pick<T>(ctx);
+    if (!sh.gi) return PF_OK;
+    const void* kern = sr ? res_kernel<T, true>(sh) : res_kernel<T, false>(sh);
+    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return PF_OK;
+    }
+    const long halo = 2 * ctx->nn * 4;
+    const bool fresh = !ctx->res_halo;
+    if (fresh) PF_TRY(dalloc(ctx, &ctx->res_halo, halo));
+    if (fresh || ctx->res_tag > 0xf0000000u) {
+        // no word may carry a tag that is still to come
+        k_fill<u64><<<gsize(halo), kBlock, 0, ctx->stream>>>(halo, ctx->res_halo, 0ull);
+        k_fill<u64><<<1, kBlock, 0, ctx->stream>>>(2L * 4 * kResMaxWg * 2, ctx->res_slots, 0ull);
+        ctx->res_tag = 1;
+    }
+    PcgDev* S = (PcgDev*)ctx->d_pcg;
+    k_res_start<<<1, 1, 0, ctx->stream>>>(S, ctx->d_res);
+    PF_TRY(check_launch(ctx));
+    const bool f32 = std::is_same<T, float>::value;
+    ResArgs<T> A{};
+    A.nx = ctx->nx; A.ny = ctx->ny; A.gi = sh.gi; A.gj = sh.gj;
+    A.b = b; A.D = D;
+    A.E = f32 ? (const T*)ctx->d_Ef : (const T*)ctx->d_E;
+    A.K0 = f32 ? (const T*)ctx->d_K0f : (const T*)ctx->d_K0;
+    A.x = x; A.r = r; A.s = s; A.p = p; A.w = w;
+    A.fix = ctx->d_fix;
+    A.slots = ctx->res_slots; A.halo = ctx->res_halo;
+    A.S = S; A.R = ctx->d_res;
+    A.eps = eps;
+    const long end = sr ? (long)itrmax + 1 : itrmax;  // sr: step m finishes iterate m
+    const PcgDev* H = (const PcgDev*)ctx->h_pcg;
+    for (long m = 0;;) {
+        A.m0 = (int)m;
+        A.m1 = (int)std::min(end, m + kResChunk);
+        A.last = A.m1 == end;
+        A.tag = ctx->res_tag;
+        ctx->res_tag += 2 * (A.m1 - A.m0) + 2;
+        void* args[] = {&A};
+        if (hipLaunchCooperativeKernel(kern, dim3(sh.gi * sh.gj), dim3(sh.nt), args, (unsigned)sh.lds, ctx->stream) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            if (m == 0) return PF_OK;
+            ctx->err = "hipLaunchCooperativeKernel failed inside a resident solve";
+            return PF_ERR_HIP;
+        }
+        PF_HIP(hipMemcpyAsync(ctx->h_pcg, S, sizeof(PcgDev), hipMemcpyDeviceToHost, ctx->stream));
+        PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
+        PF_TRY(sync(ctx));
+        if (((const ResDev*)ctx->h_res)->stall) {
+            ctx->res_stalled = true;
+            return PF_OK;
+        }
+        m = A.m1;
+        if (H->done || m >= end) break;
+    }
+    *ran = true;
+    out.iterations = H->iterations;
+    out.status = H->status;
+    out.rnorm = H->rnorm;
+    out.bnorm = H->bnorm;
+    return PF_OK;
+}
+
 // Workgroups of k_cg1_q4_tile: full tiles, then edge tiles (launched first).
 Cg1Tiles cg1_tiles(const pf_ctx* ctx, unsigned* grid, int ti = kCg1TI, int tj = kCg1TJ) {
     Cg1Tiles G;
@@ -450,8 +585,13 @@ int pcg_device_cg1(pf_ctx* ctx, const T* b, T* x, const T* D, T* r, T* z, T* p0,
     T* W[2] = {p1, q};
     T* Sv[2] = {s0, s1};
     T* Dinv = (T*)ctx->d_Dinv;
-    k_cg1_start<<<1, 1, 0, ctx->stream>>>(S);
     k_recip<T><<<gsize(ctx->nv), kBlock, 0, ctx->stream>>>(ctx->nv, D, Dinv);
+    if (ctx->pcg_form != PF_PCG_SINGLE_REDUCTION_RECOMPUTED) {
+        bool ran;
+        PF_TRY(pcg_resident<T>(ctx, true, b, x, Dinv, r, s0, p0, q, eps, itrmax, out, &ran));
+        if (ran) return PF_OK;
+    }
+    k_cg1_start<<<1, 1, 0, ctx->stream>>>(S);
     PF_TRY(check_launch(ctx));
     const int chunk = 32;
     const int mmax = itrmax + 1;  // launch m finishes iterate m; iterate itrmax is the last
@@ -513,6 +653,11 @@ int pcg_device(pf_ctx* ctx, bool csr, const T* b, T* x, const T* D, T* r, T* z, 
     // drifts and the single-reduction form needs about a third more iterations
     if (!csr && is2d(ctx) && ctx->pcg_form != PF_PCG_SCALINGCG && !snap && std::is_same<T, double>::value)
         return pcg_device_cg1<T>(ctx, b, x, D, r, z, p0, p1, q, eps, itrmax, out);
+    if (!csr && is2d(ctx) && !snap) {
+        bool ran;
+        PF_TRY(pcg_resident<T>(ctx, false, b, x, D, r, z, p0, q, eps, itrmax, out, &ran));
+        if (ran) return PF_OK;
+    }
     const long n = csr ? ctx->N : ctx->nv;
     PcgDev* S = (PcgDev*)ctx->d_pcg;
     double* partA = ctx->red.partials;
@@ -2767,16 +2912,32 @@ int pf_create(pf_ctx** out, int device) {
     ctx->device = device;
     int rc = set_device(ctx);
     if (rc == PF_OK && hipStreamCreate(&ctx->stream) != hipSuccess) rc = PF_ERR_HIP;
-    if (rc == PF_OK) rc = dalloc(ctx, &ctx->red.partials, 8L * kMaxPartials);
+    // the partial sums, then the resident solves' slots and scalars
+    constexpr long kResWords = 2L * 4 * kResMaxWg * 2;
+    static_assert(sizeof(ResDev) % 8 == 0, "whole words");
+    if (rc == PF_OK)
+        rc = dalloc(ctx, &ctx->red.partials, 8L * kMaxPartials + kResWords + (long)sizeof(ResDev) / 8);
+    if (rc == PF_OK) {
+        ctx->res_slots = (u64*)(ctx->red.partials + 8L * kMaxPartials);
+        ctx->d_res = (ResDev*)(ctx->res_slots + kResWords);
+    }
     if (rc == PF_OK) rc = dalloc(ctx, &ctx->red.counter, 1);
     if (rc == PF_OK) rc = dalloc(ctx, &ctx->red.out, 16);
     if (rc == PF_OK && hipMalloc((void**)&ctx->d_pcg, sizeof(PcgDev)) != hipSuccess) rc = PF_ERR_NOMEM;
     if (rc == PF_OK && hipMalloc((void**)&ctx->d_oc, sizeof(OcDev)) != hipSuccess) rc = PF_ERR_NOMEM;
     if (rc == PF_OK && hipHostMalloc((void**)&ctx->h_pcg, sizeof(PcgDev)) != hipSuccess) rc = PF_ERR_NOMEM;
     if (rc == PF_OK && hipHostMalloc((void**)&ctx->h_oc, sizeof(OcDev)) != hipSuccess) rc = PF_ERR_NOMEM;
-    if (rc == PF_OK && hipHostMalloc((void**)&ctx->h_red, sizeof(double) * 16) != hipSuccess) rc = PF_ERR_NOMEM;
+    if (rc == PF_OK && hipHostMalloc((void**)&ctx->h_red, sizeof(double) * 16 + sizeof(ResDev)) != hipSuccess)
+        rc = PF_ERR_NOMEM;
+    if (rc == PF_OK) ctx->h_res = (ResDev*)(ctx->h_red + 16);
     if (rc == PF_OK && hipMemset(ctx->d_pcg, 0, sizeof(PcgDev)) != hipSuccess) rc = PF_ERR_HIP;
     if (rc == PF_OK) rc = noalloc_scratch_init(ctx);
+    if (rc == PF_OK) {
+        int coop = 0, cus = 0;
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device);
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+        ctx->res_wgs = coop ? std::min(cus, kResMaxWg) : 0;
+    }
     if (rc != PF_OK) {
         pf_destroy(ctx);
         return rc;

@@ -28,12 +28,13 @@ constexpr int kMaxPartials = 8192;  // upper bound on workgroups of a reducing l
 // write them, pf_kernels.hip) and of the OC bisection.
 struct PcgDev;
 struct OcDev;
+struct ResDev;
 
 // Reduction scratch: per-workgroup partials and the arrival counter of the
 // "last workgroup reduces" pattern.  One set per context; launches that reduce
 // are serialised on the context's stream.
 struct ReduceScratch {
-    double* partials;    // kMaxPartials * 4 doubles
+    double* partials;    // kMaxPartials * 8 doubles, then the resident solves' slots and scalars
     unsigned* counter;   // one counter, returned to zero by the last workgroup
     double* out;         // 16 doubles of results
 };
@@ -117,6 +118,16 @@ struct pf_ctx {
     pf::PcgDev* h_pcg = nullptr;  // pinned mirror
     pf::OcDev* h_oc = nullptr;    // pinned mirror
     double* h_red = nullptr;          // pinned mirror of red.out
+
+    // resident solves (pf_resident.hip): exchange buffers and scalars between
+    // launches (slots, d_res and h_res are parts of red.partials and h_red),
+    // the next unused exchange tag, the workgroups that run at once (0: none),
+    // and whether a solve stalled (this context then launches)
+    unsigned long long *res_slots = nullptr, *res_halo = nullptr;
+    pf::ResDev *d_res = nullptr, *h_res = nullptr;
+    unsigned res_tag = 1;
+    int res_wgs = 0;
+    bool res_stalled = false;
 
     // MMA state
     struct MmaState* mma = nullptr;

@@ -62,13 +62,13 @@ __global__ void k_convert(long n, const A* __restrict__ a, B* __restrict__ b) {
 template <class T>
 struct alignas(2 * sizeof(T)) Vec2 { T x, y; };
 
-template <class T>
-__device__ inline void elem_rows_q4(const T* __restrict__ K0, int loc, const Vec2<T> n0, const Vec2<T> n1,
+template <class T, class KP>
+__device__ inline void elem_rows_q4(KP K0, int loc, const Vec2<T> n0, const Vec2<T> n1,
                                     const Vec2<T> n2, const Vec2<T> n3, T& ox, T& oy) {
 #pragma clang fp contract(fast)  // not a check-path kernel: FMA allowed
     // rows 2*loc, 2*loc+1 of K0 times the element vector (BL, BR, TR, TL)
-    const T* r0 = K0 + (2 * loc) * 8;
-    const T* r1 = r0 + 8;
+    const KP r0 = K0 + (2 * loc) * 8;
+    const KP r1 = r0 + 8;
     T a = 0, b = 0;
     a += r0[0] * n0.x; a += r0[1] * n0.y; a += r0[2] * n1.x; a += r0[3] * n1.y;
     a += r0[4] * n2.x; a += r0[5] * n2.y; a += r0[6] * n3.x; a += r0[7] * n3.y;
@@ -85,22 +85,22 @@ __device__ inline void apply_q4_node(int nx, int ny, int i, int j, const Vec2<T>
     T ax = 0, ay = 0, ex, ey;
     if (i >= 1 && j >= 1) {  // element (i-1, j-1): this node is TR
         T Ee = E[(long)ny * (i - 1) + (j - 1)];
-        elem_rows_q4(K0, 2, v[0][0], v[1][0], v[1][1], v[0][1], ex, ey);
+        elem_rows_q4<T>(K0, 2, v[0][0], v[1][0], v[1][1], v[0][1], ex, ey);
         ax += Ee * ex; ay += Ee * ey;
     }
     if (i >= 1 && j < ny) {  // element (i-1, j): BR
         T Ee = E[(long)ny * (i - 1) + j];
-        elem_rows_q4(K0, 1, v[0][1], v[1][1], v[1][2], v[0][2], ex, ey);
+        elem_rows_q4<T>(K0, 1, v[0][1], v[1][1], v[1][2], v[0][2], ex, ey);
         ax += Ee * ex; ay += Ee * ey;
     }
     if (i < nx && j >= 1) {  // element (i, j-1): TL
         T Ee = E[(long)ny * i + (j - 1)];
-        elem_rows_q4(K0, 3, v[1][0], v[2][0], v[2][1], v[1][1], ex, ey);
+        elem_rows_q4<T>(K0, 3, v[1][0], v[2][0], v[2][1], v[1][1], ex, ey);
         ax += Ee * ex; ay += Ee * ey;
     }
     if (i < nx && j < ny) {  // element (i, j): BL
         T Ee = E[(long)ny * i + j];
-        elem_rows_q4(K0, 0, v[1][1], v[2][1], v[2][2], v[1][2], ex, ey);
+        elem_rows_q4<T>(K0, 0, v[1][1], v[2][1], v[2][2], v[1][2], ex, ey);
         ax += Ee * ex; ay += Ee * ey;
     }
     yx = ax;
@@ -388,22 +388,22 @@ __global__ void __launch_bounds__(256) k_pcg_k1_q4_tile(int nx, int ny, int tile
             if (i > nx || j > ny) continue;
             T ax = 0, ay = 0, ex, ey;
             if (i >= 1 && j >= 1) {  // element (i-1, j-1): this node is TR
-                elem_rows_q4(K0, 2, sp[r][c], sp[r + 1][c], sp[r + 1][c + 1], sp[r][c + 1], ex, ey);
+                elem_rows_q4<T>(K0, 2, sp[r][c], sp[r + 1][c], sp[r + 1][c + 1], sp[r][c + 1], ex, ey);
                 T Ee = se[r][c];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i >= 1 && j < ny) {  // element (i-1, j): BR
-                elem_rows_q4(K0, 1, sp[r][c + 1], sp[r + 1][c + 1], sp[r + 1][c + 2], sp[r][c + 2], ex, ey);
+                elem_rows_q4<T>(K0, 1, sp[r][c + 1], sp[r + 1][c + 1], sp[r + 1][c + 2], sp[r][c + 2], ex, ey);
                 T Ee = se[r][c + 1];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i < nx && j >= 1) {  // element (i, j-1): TL
-                elem_rows_q4(K0, 3, sp[r + 1][c], sp[r + 2][c], sp[r + 2][c + 1], sp[r + 1][c + 1], ex, ey);
+                elem_rows_q4<T>(K0, 3, sp[r + 1][c], sp[r + 2][c], sp[r + 2][c + 1], sp[r + 1][c + 1], ex, ey);
                 T Ee = se[r + 1][c];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i < nx && j < ny) {  // element (i, j): BL
-                elem_rows_q4(K0, 0, sp[r + 1][c + 1], sp[r + 2][c + 1], sp[r + 2][c + 2], sp[r + 1][c + 2], ex, ey);
+                elem_rows_q4<T>(K0, 0, sp[r + 1][c + 1], sp[r + 2][c + 1], sp[r + 2][c + 2], sp[r + 1][c + 2], ex, ey);
                 T Ee = se[r + 1][c + 1];
                 ax += Ee * ex; ay += Ee * ey;
             }
@@ -706,22 +706,22 @@ __global__ void __launch_bounds__(256) k_cg1_q4_tile(int nx, int ny, Cg1Tiles G,
             if (i > nx || j > ny) continue;
             T ax = 0, ay = 0, ex, ey;
             if (i >= 1 && j >= 1) {  // element (i-1, j-1): this node is TR
-                elem_rows_q4(K0, 2, v[o][0], v[o + 1][0], v[o + 1][1], v[o][1], ex, ey);
+                elem_rows_q4<T>(K0, 2, v[o][0], v[o + 1][0], v[o + 1][1], v[o][1], ex, ey);
                 const T Ee = em[o][0];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i >= 1 && j < ny) {  // element (i-1, j): BR
-                elem_rows_q4(K0, 1, v[o][1], v[o + 1][1], v[o + 1][2], v[o][2], ex, ey);
+                elem_rows_q4<T>(K0, 1, v[o][1], v[o + 1][1], v[o + 1][2], v[o][2], ex, ey);
                 const T Ee = em[o][1];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i < nx && j >= 1) {  // element (i, j-1): TL
-                elem_rows_q4(K0, 3, v[o + 1][0], v[o + 2][0], v[o + 2][1], v[o + 1][1], ex, ey);
+                elem_rows_q4<T>(K0, 3, v[o + 1][0], v[o + 2][0], v[o + 2][1], v[o + 1][1], ex, ey);
                 const T Ee = em[o + 1][0];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i < nx && j < ny) {  // element (i, j): BL
-                elem_rows_q4(K0, 0, v[o + 1][1], v[o + 2][1], v[o + 2][2], v[o + 1][2], ex, ey);
+                elem_rows_q4<T>(K0, 0, v[o + 1][1], v[o + 2][1], v[o + 2][2], v[o + 1][2], ex, ey);
                 const T Ee = em[o + 1][1];
                 ax += Ee * ex; ay += Ee * ey;
             }
@@ -908,22 +908,22 @@ __global__ void __launch_bounds__(256) k_cg2_q4_tile(int nx, int ny, Cg1Tiles G,
             T ax = 0, ay = 0, ex, ey;
             if (prev) {  // s = K p (alpha = 0 at launch 0)
                 if (ii >= 1 && jj >= 1) {
-                    elem_rows_q4(K0, 2, s0[0], s0[w2], s0[w2 + 1], s0[1], ex, ey);
+                    elem_rows_q4<T>(K0, 2, s0[0], s0[w2], s0[w2 + 1], s0[1], ex, ey);
                     const T Ee = se[a * we + b];
                     ax += Ee * ex; ay += Ee * ey;
                 }
                 if (ii >= 1 && jj < ny) {
-                    elem_rows_q4(K0, 1, s0[1], s0[w2 + 1], s0[w2 + 2], s0[2], ex, ey);
+                    elem_rows_q4<T>(K0, 1, s0[1], s0[w2 + 1], s0[w2 + 2], s0[2], ex, ey);
                     const T Ee = se[a * we + b + 1];
                     ax += Ee * ex; ay += Ee * ey;
                 }
                 if (ii < nx && jj >= 1) {
-                    elem_rows_q4(K0, 3, s0[w2], s0[2 * w2], s0[2 * w2 + 1], s0[w2 + 1], ex, ey);
+                    elem_rows_q4<T>(K0, 3, s0[w2], s0[2 * w2], s0[2 * w2 + 1], s0[w2 + 1], ex, ey);
                     const T Ee = se[(a + 1) * we + b];
                     ax += Ee * ex; ay += Ee * ey;
                 }
                 if (ii < nx && jj < ny) {
-                    elem_rows_q4(K0, 0, s0[w2 + 1], s0[2 * w2 + 1], s0[2 * w2 + 2], s0[w2 + 2], ex, ey);
+                    elem_rows_q4<T>(K0, 0, s0[w2 + 1], s0[2 * w2 + 1], s0[2 * w2 + 2], s0[w2 + 2], ex, ey);
                     const T Ee = se[(a + 1) * we + b + 1];
                     ax += Ee * ex; ay += Ee * ey;
                 }
@@ -968,22 +968,22 @@ __global__ void __launch_bounds__(256) k_cg2_q4_tile(int nx, int ny, Cg1Tiles G,
             const Vec2<T>* s0 = su + r * w1 + c;  // R1 rows r, r+1, r+2 from column c
             T ax = 0, ay = 0, ex, ey;
             if (i >= 1 && j >= 1) {
-                elem_rows_q4(K0, 2, s0[0], s0[w1], s0[w1 + 1], s0[1], ex, ey);
+                elem_rows_q4<T>(K0, 2, s0[0], s0[w1], s0[w1 + 1], s0[1], ex, ey);
                 const T Ee = se[(r + 1) * we + c + 1];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i >= 1 && j < ny) {
-                elem_rows_q4(K0, 1, s0[1], s0[w1 + 1], s0[w1 + 2], s0[2], ex, ey);
+                elem_rows_q4<T>(K0, 1, s0[1], s0[w1 + 1], s0[w1 + 2], s0[2], ex, ey);
                 const T Ee = se[(r + 1) * we + c + 2];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i < nx && j >= 1) {
-                elem_rows_q4(K0, 3, s0[w1], s0[2 * w1], s0[2 * w1 + 1], s0[w1 + 1], ex, ey);
+                elem_rows_q4<T>(K0, 3, s0[w1], s0[2 * w1], s0[2 * w1 + 1], s0[w1 + 1], ex, ey);
                 const T Ee = se[(r + 2) * we + c + 1];
                 ax += Ee * ex; ay += Ee * ey;
             }
             if (i < nx && j < ny) {
-                elem_rows_q4(K0, 0, s0[w1 + 1], s0[2 * w1 + 1], s0[2 * w1 + 2], s0[w1 + 2], ex, ey);
+                elem_rows_q4<T>(K0, 0, s0[w1 + 1], s0[2 * w1 + 1], s0[2 * w1 + 2], s0[w1 + 2], ex, ey);
                 const T Ee = se[(r + 2) * we + c + 2];
                 ax += Ee * ex; ay += Ee * ey;
             }
