@@ -219,6 +219,10 @@ int pf_set_pcg_form(pf_ctx* ctx, int form);
  *   PF_H8_OP_MFMA: the element matrix as a batched product on the matrix
  *     cores (16 elements of one colour per product, K0 in registers), the
  *     rows summed per node in LDS in colour order (deterministic).
+ * Until a call chooses one, Jacobi-PCG solves of grids that fit the chip (up
+ * to about 128 x 64 x 64 elements) run in one resident kernel, with the
+ * element matrix in its parity basis where it has one (any box element of a
+ * material with the box's mirror planes), and the others use PF_H8_OP_VALU.
  * Has no counterpart in the reference. */
 enum { PF_H8_OP_VALU = 0, PF_H8_OP_MFMA = 1 };
 int pf_set_h8_operator(pf_ctx* ctx, int kind);

@@ -1,18 +1,20 @@
 // C-ABI of libpansfem2_amd: context, grids, DOF maps, operators, solvers,
 // filter, OC and the device-resident SIMP loop.  Declarations and the
 // reference routine each entry point replaces: include/pansfem2_amd.h.
+#include <algorithm>
+#include <cmath>
+
 #include "pf_kernels.hip"
 #include "pf_resident.hip"
 #include "pf_mma.hip"
 #include "pf_hex8.hip"
+#include "pf_resident3.hip"
 #include "pf_learned.hip"
 #include "pf_mg.hip"
 #include "pf_mg3.hip"
 
-#include <algorithm>
 #include <chrono>
 #include <type_traits>
-#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -255,6 +257,8 @@ void free_grid(pf_ctx* ctx) {
     dfree(ctx->d_s0); dfree(ctx->d_s1); dfree(ctx->f_s0); dfree(ctx->f_s1); dfree(ctx->d_Dinv);
     dfree(ctx->f_D); dfree(ctx->f_b);
     dfree(ctx->res_halo);
+    dfree(ctx->res_loc);
+    ctx->res_halo_n = ctx->res_loc_n = 0;
     dfree(ctx->d_e0); dfree(ctx->d_e1); dfree(ctx->d_e2); dfree(ctx->d_e3); dfree(ctx->d_e4); dfree(ctx->d_e5);
     dfree(ctx->d_e6);
     dfree(ctx->d_cg); dfree(ctx->d_load);
@@ -470,47 +474,36 @@ const void* res_kernel(const ResShape& sh) {
     return nullptr;
 }
 
-// Jacobi-PCG resident on the chip (k_pcg_q4_resident); *ran is false, and
-// nothing has been solved, when the grid does not fit or the launch cannot be
-// made or stalled: the caller then launches per iteration.  D: the diagonal,
-// or its inverse for the single-reduction form (sr).
 constexpr int kResChunk = 2048;  // iterations per launch: other streams get the GPU in between
-template <class T>
-int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s, T* p, T* w, double eps, int itrmax,
-                 PcgRun& out, bool* ran) {
-    *ran = false;
-    if (ctx->res_wgs < 1 || ctx->res_stalled) return PF_OK;
-    const ResShape sh = res_pick<T>(ctx);
-    if (!sh.gi) return PF_OK;
-    const void* kern = sr ? res_kernel<T, true>(sh) : res_kernel<T, false>(sh);
-    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds) != hipSuccess) {
-        (void)hipGetLastError();
-        return PF_OK;
+
+// Exchange buffer of `words` words for a solve that starts now, and the
+// solve's scalars.
+int res_begin(pf_ctx* ctx, long words) {
+    const bool fresh = ctx->res_halo_n < words;
+    if (fresh) {
+        ctx->res_halo_n = 0;
+        PF_TRY(dalloc(ctx, &ctx->res_halo, words));
+        ctx->res_halo_n = words;
     }
-    const long halo = 2 * ctx->nn * 4;
-    const bool fresh = !ctx->res_halo;
-    if (fresh) PF_TRY(dalloc(ctx, &ctx->res_halo, halo));
     if (fresh || ctx->res_tag > 0xf0000000u) {
         // no word may carry a tag that is still to come
-        k_fill<u64><<<gsize(halo), kBlock, 0, ctx->stream>>>(halo, ctx->res_halo, 0ull);
+        k_fill<u64><<<gsize(words), kBlock, 0, ctx->stream>>>(ctx->res_halo_n, ctx->res_halo, 0ull);
         k_fill<u64><<<1, kBlock, 0, ctx->stream>>>(2L * 4 * kResMaxWg * 2, ctx->res_slots, 0ull);
         ctx->res_tag = 1;
     }
-    PcgDev* S = (PcgDev*)ctx->d_pcg;
-    k_res_start<<<1, 1, 0, ctx->stream>>>(S, ctx->d_res);
-    PF_TRY(check_launch(ctx));
-    const bool f32 = std::is_same<T, float>::value;
-    ResArgs<T> A{};
-    A.nx = ctx->nx; A.ny = ctx->ny; A.gi = sh.gi; A.gj = sh.gj;
-    A.b = b; A.D = D;
-    A.E = f32 ? (const T*)ctx->d_Ef : (const T*)ctx->d_E;
-    A.K0 = f32 ? (const T*)ctx->d_K0f : (const T*)ctx->d_K0;
-    A.x = x; A.r = r; A.s = s; A.p = p; A.w = w;
+    k_res_start<<<1, 1, 0, ctx->stream>>>((PcgDev*)ctx->d_pcg, ctx->d_res);
+    return check_launch(ctx);
+}
+
+// Launches `kern` (cooperatively) over iterations 0 .. end in chunks until the
+// solve is done; *ran is false, and nothing has been solved, when the launch
+// cannot be made or stalled: the caller then launches per iteration.
+template <class ARGS>
+int res_run(pf_ctx* ctx, const void* kern, int wgs, int nt, size_t lds, ARGS& A, long end, PcgRun& out, bool* ran) {
+    A.slots = ctx->res_slots;
+    A.S = (PcgDev*)ctx->d_pcg;
+    A.R = ctx->d_res;
     A.fix = ctx->d_fix;
-    A.slots = ctx->res_slots; A.halo = ctx->res_halo;
-    A.S = S; A.R = ctx->d_res;
-    A.eps = eps;
-    const long end = sr ? (long)itrmax + 1 : itrmax;  // sr: step m finishes iterate m
     const PcgDev* H = (const PcgDev*)ctx->h_pcg;
     for (long m = 0;;) {
         A.m0 = (int)m;
@@ -519,17 +512,16 @@ int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s,
         A.tag = ctx->res_tag;
         ctx->res_tag += 2 * (A.m1 - A.m0) + 2;
         void* args[] = {&A};
-        if (hipLaunchCooperativeKernel(kern, dim3(sh.gi * sh.gj), dim3(sh.nt), args, (unsigned)sh.lds, ctx->stream) !=
-            hipSuccess) {
+        if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(nt), args, (unsigned)lds, ctx->stream) != hipSuccess) {
             (void)hipGetLastError();
             if (m == 0) return PF_OK;
             ctx->err = "hipLaunchCooperativeKernel failed inside a resident solve";
             return PF_ERR_HIP;
         }
-        PF_HIP(hipMemcpyAsync(ctx->h_pcg, S, sizeof(PcgDev), hipMemcpyDeviceToHost, ctx->stream));
+        PF_HIP(hipMemcpyAsync(ctx->h_pcg, A.S, sizeof(PcgDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_TRY(sync(ctx));
-        if (((const ResDev*)ctx->h_res)->stall) {
+        if (ctx->h_res->stall) {
             ctx->res_stalled = true;
             return PF_OK;
         }
@@ -542,6 +534,121 @@ int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s,
     out.rnorm = H->rnorm;
     out.bnorm = H->bnorm;
     return PF_OK;
+}
+
+// LDS beyond the default limit; false: the kernel cannot have it
+bool res_lds_ok(const void* kern, size_t lds) {
+    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+// Jacobi-PCG on a quad4 grid resident on the chip (k_pcg_q4_resident); *ran as
+// in res_run, also false when the grid does not fit.  D: the diagonal, or its
+// inverse for the single-reduction form (sr).
+template <class T>
+int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s, T* p, T* w, double eps, int itrmax,
+                 PcgRun& out, bool* ran) {
+    *ran = false;
+    if (ctx->res_wgs < 1 || ctx->res_stalled) return PF_OK;
+    const ResShape sh = res_pick<T>(ctx);
+    if (!sh.gi) return PF_OK;
+    const void* kern = sr ? res_kernel<T, true>(sh) : res_kernel<T, false>(sh);
+    if (!res_lds_ok(kern, sh.lds)) return PF_OK;
+    PF_TRY(res_begin(ctx, 2 * ctx->nn * 4));
+    const bool f32 = std::is_same<T, float>::value;
+    ResArgs<T> A{};
+    A.nx = ctx->nx; A.ny = ctx->ny; A.gi = sh.gi; A.gj = sh.gj;
+    A.b = b; A.D = D;
+    A.E = f32 ? (const T*)ctx->d_Ef : (const T*)ctx->d_E;
+    A.K0 = f32 ? (const T*)ctx->d_K0f : (const T*)ctx->d_K0;
+    A.x = x; A.r = r; A.s = s; A.p = p; A.w = w;
+    A.halo = ctx->res_halo;
+    A.eps = eps;
+    // sr: step m finishes iterate m
+    return res_run(ctx, kern, sh.gi * sh.gj, sh.nt, sh.lds, A, sr ? (long)itrmax + 1 : itrmax, out, ran);
+}
+
+// Boxes of a hex8 resident solve.  gi == 0: the grid does not fit.
+struct Res3Shape {
+    int gi = 0, gj = 0, gk = 0, slots = 0, box = 0, fb[3] = {0, 0, 0};
+    size_t lds = 0;
+};
+// The split with the least estimated time per iteration in microseconds:
+// 1.5 per pass over a layer of each half box (two waves per SIMD from 9 element
+// rows on), 0.001 per node value, 1.8 per split axis (an exchange), 0.0008 per
+// exchanged face value.  60x30x30: 30x4x2 boxes 13.2, 15x4x4 15.0, 12x3x3 21.0;
+// 128x64x64: 16x4x4 31.6, 8x8x4 39 to 44.
+template <class T>
+Res3Shape res3_pick(const pf_ctx* ctx) {
+    Res3Shape best;
+    double bestc = 0.0;
+    for (int gi = 1; gi <= std::min(ctx->nx, ctx->res_wgs); gi++)
+        for (int gj = 1; gj <= std::min(ctx->ny, ctx->res_wgs / gi); gj++)
+            for (int gk = 1; gk <= std::min(ctx->nz, ctx->res_wgs / (gi * gj)); gk++) {
+                const int ei = (ctx->nx + gi - 1) / gi, ej = (ctx->ny + gj - 1) / gj, ek = (ctx->nz + gk - 1) / gk;
+                const int di = ei + 1, dj = ej + 1, dk = ek + 1;
+                const long nv = 3L * di * dj * dk;
+                if (ej > 16 || ek > 16 || nv > kRes3Threads * kRes3Slots) continue;
+                int box = 0, most = 0, fb[3];
+                for (int ax = 0; ax < 3; ax++) {
+                    const int F = res3_face(ax, di, dj, dk);
+                    fb[ax] = box;
+                    box += 2 * F * (int)(sizeof(T) / 4);
+                    most = std::max(most, 2 * F);
+                }
+                if (most > kRes3Threads * kRes3Items) continue;
+                double cost = 1.5 * ((ei + 1) / 2 + 1) * (ej > 8 ? 1.5 : 1.0) + 0.001 * nv;
+                const int gd[3] = {gi, gj, gk};
+                for (int ax = 0; ax < 3; ax++)
+                    if (gd[ax] > 1) cost += 1.8 + 0.0008 * 2 * res3_face(ax, di, dj, dk);
+                if (best.gi && cost >= bestc) continue;
+                bestc = cost;
+                best.gi = gi;
+                best.gj = gj;
+                best.gk = gk;
+                best.slots = nv <= kRes3Threads * 4 ? 4 : kRes3Slots;
+                best.box = box;
+                std::copy(fb, fb + 3, best.fb);
+                best.lds = sizeof(T) * 2 * kRes3Threads * best.slots;
+            }
+    return best;
+}
+
+// The same for hex8 (k_pcg_h8_resident), ScalingCG's order; only for an
+// element matrix with parity blocks and the default operator.
+template <class T>
+int pcg_resident3(pf_ctx* ctx, const T* b, T* x, const T* D, T* r, T* p, double eps, int itrmax, PcgRun& out,
+                  bool* ran) {
+    *ran = false;
+    if (ctx->res_wgs < 1 || ctx->res_stalled || !ctx->d_K0p || ctx->h8_op >= 0) return PF_OK;
+    const Res3Shape sh = res3_pick<T>(ctx);
+    if (!sh.gi) return PF_OK;
+    const void* kern = sh.slots == 4 ? (const void*)k_pcg_h8_resident<T, 4>
+                                     : (const void*)k_pcg_h8_resident<T, kRes3Slots>;
+    if (!res_lds_ok(kern, sh.lds)) return PF_OK;
+    const int wgs = sh.gi * sh.gj * sh.gk;
+    PF_TRY(res_begin(ctx, 2L * wgs * sh.box));
+    const long local = (long)wgs * kRes3Threads * sh.slots;  // x of every workgroup's values
+    if (ctx->res_loc_n < local) {
+        ctx->res_loc_n = 0;
+        PF_TRY(dalloc(ctx, &ctx->res_loc, local));
+        ctx->res_loc_n = local;
+    }
+    const bool f32 = std::is_same<T, float>::value;
+    Res3Args<T> A{};
+    A.nx = ctx->nx; A.ny = ctx->ny; A.nz = ctx->nz;
+    A.gi = sh.gi; A.gj = sh.gj; A.gk = sh.gk;
+    A.box = sh.box;
+    std::copy(sh.fb, sh.fb + 3, A.fb);
+    A.b = b; A.D = D;
+    A.E = f32 ? (const T*)ctx->d_Ef : (const T*)ctx->d_E;
+    A.Kp = f32 ? (const T*)ctx->d_K0pf : (const T*)ctx->d_K0p;
+    A.x = x; A.r = r; A.p = p;
+    A.edge = ctx->res_halo;
+    A.loc = (T*)ctx->res_loc;
+    A.eps = eps;
+    return res_run(ctx, kern, wgs, kRes3Threads, sh.lds, A, itrmax, out, ran);
 }
 
 // Workgroups of k_cg1_q4_tile: full tiles, then edge tiles (launched first).
@@ -653,9 +760,10 @@ int pcg_device(pf_ctx* ctx, bool csr, const T* b, T* x, const T* D, T* r, T* z, 
     // drifts and the single-reduction form needs about a third more iterations
     if (!csr && is2d(ctx) && ctx->pcg_form != PF_PCG_SCALINGCG && !snap && std::is_same<T, double>::value)
         return pcg_device_cg1<T>(ctx, b, x, D, r, z, p0, p1, q, eps, itrmax, out);
-    if (!csr && is2d(ctx) && !snap) {
+    if (!csr && !snap) {
         bool ran;
-        PF_TRY(pcg_resident<T>(ctx, false, b, x, D, r, z, p0, q, eps, itrmax, out, &ran));
+        if (is2d(ctx)) PF_TRY(pcg_resident<T>(ctx, false, b, x, D, r, z, p0, q, eps, itrmax, out, &ran));
+        else PF_TRY(pcg_resident3<T>(ctx, b, x, D, r, p0, eps, itrmax, out, &ran));
         if (ran) return PF_OK;
     }
     const long n = csr ? ctx->N : ctx->nv;
@@ -2960,6 +3068,8 @@ int pf_destroy(pf_ctx* ctx) {
     dfree(ctx->d_K0gf);
     dfree(ctx->d_K0m);
     dfree(ctx->d_K0mf);
+    dfree(ctx->d_K0p);
+    dfree(ctx->d_K0pf);
     dfree(ctx->red.partials);
     dfree(ctx->red.counter);
     dfree(ctx->red.out);
@@ -3088,6 +3198,17 @@ int pf_set_element_matrix(pf_ctx* ctx, const double* K0, int nd) {
         // the MFMA operator's A fragments
         std::vector<double> m64(768);
         std::vector<float> m32(768);
+        double par[kH8ParityCoefs];
+        float par32[kH8ParityCoefs];
+        dfree(ctx->d_K0p);
+        dfree(ctx->d_K0pf);
+        if (h8_parity_pack(K0, par)) {
+            for (int i = 0; i < kH8ParityCoefs; i++) par32[i] = (float)par[i];
+            PF_TRY(dalloc(ctx, &ctx->d_K0p, kH8ParityCoefs));
+            PF_TRY(dalloc(ctx, &ctx->d_K0pf, kH8ParityCoefs));
+            PF_HIP(hipMemcpy(ctx->d_K0p, par, sizeof(par), hipMemcpyHostToDevice));
+            PF_HIP(hipMemcpy(ctx->d_K0pf, par32, sizeof(par32), hipMemcpyHostToDevice));
+        }
         h8m_pack_k0(K0, m64.data());
         h8m_pack_k0(K0, m32.data());
         PF_TRY(dalloc(ctx, &ctx->d_K0m, 768));

@@ -68,6 +68,8 @@ struct pf_ctx {
     float* d_K0gf = nullptr;
     double* d_K0m = nullptr;  // hex8: K0 as the MFMA operator's A fragments (h8m_pack_k0)
     float* d_K0mf = nullptr;
+    double* d_K0p = nullptr;  // hex8: K0's parity blocks (h8_parity_pack); null when it has none
+    float* d_K0pf = nullptr;
 
     // material / design
     double E1 = 1.0, E0 = 1e-9, p = 3.0, nu = 0.3, t = 1.0;
@@ -124,6 +126,8 @@ struct pf_ctx {
     // the next unused exchange tag, the workgroups that run at once (0: none),
     // and whether a solve stalled (this context then launches)
     unsigned long long *res_slots = nullptr, *res_halo = nullptr;
+    double* res_loc = nullptr;              // hex8: the workgroups' own x
+    long res_halo_n = 0, res_loc_n = 0;     // their sizes
     pf::ResDev *d_res = nullptr, *h_res = nullptr;
     unsigned res_tag = 1;
     int res_wgs = 0;
@@ -139,7 +143,9 @@ struct pf_ctx {
     struct MgState* mg = nullptr;
     int mg_prolong = PF_MG_PROLONG_STIFFNESS;
     int mg_resid = PF_MG_RESIDUAL_AUTO;  // hex8 coarse-level residual form
-    int h8_op = PF_H8_OP_VALU;  // hex8 matrix-free operator of the fused PCG kernel
+    // hex8 matrix-free operator of the fused PCG kernel as pf_set_h8_operator
+    // chose it; -1, the default: the resident solve where it fits, else PF_H8_OP_VALU
+    int h8_op = -1;
 
     // device address of the library's static scratch array on this
     // context's device (pf_compliance_sens_dev_noalloc)

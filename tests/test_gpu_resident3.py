@@ -1,0 +1,90 @@
+"""GPU parity of the resident hex8 Jacobi-PCG (k_pcg_h8_resident: the element
+matrix in its parity basis, shared nodes' sums completed axis by axis) against
+the assembled-matrix solve, and the rule that decides on the parity basis.
+
+Shapes: one box, boxes of uneven sizes along every axis, one layer per half box
+and none, 16 elements along a box's edge.  The first iterates differ from the
+assembled solve's by the order of sums and the transforms' roundings: some
+hundreds of 1e-16 per entry, 1e-12 with the head room of the recurrences.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1), (2, 1, 3), (1, 5, 2), (4, 2, 2), (8, 4, 4), (17, 9, 5), (3, 18, 16), (5, 3, 37), (33, 16, 16),
+          (30, 15, 17)]
+
+
+@pytest.fixture(scope="module")
+def pa():
+    import pansfem2_amd
+    return pansfem2_amd
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def problem(pa, nx, ny, nz):
+    ctx = pa.cantilever3d(nx, ny, nz)
+    rng = np.random.default_rng(nx * 10000 + ny * 100 + nz)
+    ctx.set_density(rng.uniform(0.2, 1.0, nx * ny * nz))
+    return ctx, ctx.load() + rng.uniform(-1e-3, 1e-3, ctx.N)
+
+
+@pytest.mark.parametrize("nx,ny,nz", SHAPES)
+def test_iterates_against_assembled(pa, nx, ny, nz):
+    print(f"hex8 resident {nx}x{ny}x{nz}", flush=True)
+    ctx, b = problem(pa, nx, ny, nz)
+    ctx.assemble_csr()
+    for k in (1, 2, 6):
+        xr, sr = ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-14, itrmax=k)
+        x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-14, itrmax=k)
+        assert st["iterations"] == sr["iterations"]
+        assert rel(x, xr) < 1e-12, (k, rel(x, xr))
+    xr, sr = ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-10)
+    x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-10)
+    assert st["status"] == 1 and st["true_residual"] < 1e-9
+    assert abs(st["iterations"] - sr["iterations"]) <= max(3, 0.005 * sr["iterations"])
+    assert rel(x, xr) < 1e-8
+    assert np.array_equal(x, ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-10)[0])
+    x32, s32 = ctx.pcg(b, op=pa.PF_OP_EBE32, eps=1e-9)
+    assert s32["status"] == 1 and s32["true_residual"] <= 1.0000001e-9
+    assert rel(x32, xr) < 1e-6
+    ctx.close()
+
+
+def test_more_iterations_than_one_launch(pa):
+    ctx, _ = problem(pa, 60, 6, 5)
+    rng = np.random.default_rng(3)
+    ctx.set_density(rng.uniform(0.05, 1.0, 60 * 6 * 5))
+    b = ctx.load()
+    ctx.assemble_csr()
+    for k in (2047, 2048, 2049):
+        x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=0.0, itrmax=k)
+        assert st["iterations"] == k and st["status"] == 2
+    xr, _ = ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-11)
+    assert rel(x, xr) < 1e-7
+    ctx.close()
+
+
+def test_element_matrix_without_parity_blocks(pa):
+    """A matrix that the mirrors do not leave as it is (a sheared material), one
+    that is not symmetric and one that resists translations take the general
+    operator: the same iterates as the MFMA operator, which applies any
+    matrix.  The scaled original still takes the resident solve."""
+    rng = np.random.default_rng(7)
+    ctx, b = problem(pa, 6, 4, 5)
+    K = ctx.element_stiffness(0, 1.0, 0.3)
+    S = rng.uniform(-1, 1, (24, 24))
+    other, _ = problem(pa, 6, 4, 5)
+    other.set_h8_operator(pa.PF_H8_OP_MFMA)
+    for k0 in (K + 1e-3 * (S @ S.T) / 24, K + 1e-6 * rng.uniform(-1, 1, (24, 24)), K + 1e-3 * np.eye(24), 2.0 * K):
+        ctx.set_element_matrix(k0)
+        other.set_element_matrix(k0)
+        x = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-30, itrmax=5)[0]
+        xm = other.pcg(b, op=pa.PF_OP_EBE64, eps=1e-30, itrmax=5)[0]
+        assert rel(x, xm) < 1e-12
+    ctx.close()
+    other.close()
