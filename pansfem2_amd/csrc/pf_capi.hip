@@ -2791,23 +2791,6 @@ int host_partials(pf_ctx* ctx, const double* part, int nparts, int K, double* ou
     return PF_OK;
 }
 
-// MMA<T>::solvels for the 2x2 system (MMA.h:464-509).
-void solve2(double A[2][2], double b[2], double x[2]) {
-    double pivot = std::fabs(A[0][0]);
-    if (pivot < std::fabs(A[1][0])) {
-        std::swap(b[0], b[1]);
-        std::swap(A[0][0], A[1][0]);
-        std::swap(A[0][1], A[1][1]);
-    }
-    A[1][1] -= A[0][1] * A[1][0] / A[0][0];
-    b[1] -= b[0] * A[1][0] / A[0][0];
-    x[1] = b[1];
-    x[1] /= A[1][1];
-    x[0] = b[0];
-    x[0] -= x[1] * A[0][1];
-    x[0] /= A[0][0];
-}
-
 double max5(double a, double b, double c, double d, double e) {
     double r = a;
     if (r < b) r = b;
@@ -2815,6 +2798,72 @@ double max5(double a, double b, double c, double d, double e) {
     if (r < d) r = d;
     if (r < e) r = e;
     return r;
+}
+
+// The update in one resident launch (k_mma_resident); *ran is false, and the
+// state as it was, when the variables do not fit the registers of the chip or
+// the launch cannot be made or stalled.
+int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, const double* dgdx, int* steps,
+                        int* status, bool* ran) {
+    MmaState* M = ctx->mma;
+    const pf_mma_params& P = M->prm;
+    *ran = false;
+    const int max_newton = P.max_newton > 0 ? P.max_newton : 500;
+    constexpr int NT = kMmaResThreads;
+    const long most = (long)ctx->res_wgs * NT;
+    if (ctx->res_stalled || most <= 0 || M->n > 4 * most || max_newton > 100000) return PF_OK;
+    // one variable per thread while the workgroups last, then two, then four
+    const int S = M->n <= most ? 1 : M->n <= 2 * most ? 2 : 4;
+    const void* kern = M->conlin ? (S == 1 ? (const void*)k_mma_resident<1, true>
+                                    : S == 2 ? (const void*)k_mma_resident<2, true>
+                                             : (const void*)k_mma_resident<4, true>)
+                                 : (S == 1 ? (const void*)k_mma_resident<1, false>
+                                    : S == 2 ? (const void*)k_mma_resident<2, false>
+                                             : (const void*)k_mma_resident<4, false>);
+    PF_TRY(res_begin(ctx, 0));
+    MmaRes A{};
+    A.n = M->n;
+    A.early = M->k < 2;
+    A.max_newton = max_newton;
+    A.tag = ctx->res_tag;
+    ctx->res_tag += 1 + 52u * (unsigned)max_newton;  // two exchanges and at most 50 trials a step
+    A.a0 = P.a0; A.a = P.a; A.c = P.c; A.d = P.d;
+    A.xmin = P.xmin; A.xmax = P.xmax; A.raa0 = P.raa0; A.albefa = P.albefa; A.move = P.move;
+    A.asyinit = P.asyinit; A.asydecr = P.asydecr; A.asyincr = P.asyincr;
+    A.g = g;
+    A.xk = xk; A.xkm1 = M->xkm1; A.xkm2 = M->xkm2; A.L = M->L; A.U = M->U;
+    A.dfdx = dfdx; A.dgdx = dgdx;
+    A.xo = M->x; A.Lo = M->alpha; A.Uo = M->beta;
+    A.slots = ctx->res_slots;
+    A.R = ctx->d_res;
+    void* args[] = {&A};
+    const unsigned wgs = (unsigned)((M->n + (long)NT * S - 1) / ((long)NT * S));
+    if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(NT), args, 0, ctx->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return PF_OK;
+    }
+    PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
+    PF_TRY(sync(ctx));
+    if (ctx->h_res->stall) {
+        ctx->res_stalled = true;
+        return PF_OK;
+    }
+    *steps = (int)ctx->h_res->v[0];
+    *status = (int)ctx->h_res->v[1];
+    *ran = true;
+    return PF_OK;
+}
+
+// The new variables (M->x) and the state for the next update.
+int mma_accept(pf_ctx* ctx, double* xk, double f) {
+    MmaState* M = ctx->mma;
+    M->previousvalue = f;
+    M->k++;
+    const size_t eb = sizeof(double) * M->n;
+    std::swap(M->xkm1, M->xkm2);
+    PF_HIP(hipMemcpyAsync(M->xkm1, xk, eb, hipMemcpyDeviceToDevice, ctx->stream));
+    PF_HIP(hipMemcpyAsync(xk, M->x, eb, hipMemcpyDeviceToDevice, ctx->stream));
+    return sync(ctx);
 }
 
 // MMA<T>::UpdateVariables (MMA.h:116-419) for m = 1 on device arrays.
@@ -2825,6 +2874,24 @@ int mma_update_device(pf_ctx* ctx, double* xk, double f, const double* dfdx, dou
     const long n = M->n;
     const pf_mma_params& P = M->prm;
     const double a = P.a, c = P.c, d = P.d, a0 = P.a0;
+    {
+        int steps = 0, status = 0;
+        bool ran;
+        PF_TRY(mma_update_resident(ctx, xk, dfdx, g, dgdx, &steps, &status, &ran));
+        if (ran) {
+            if (steps_out) *steps_out = steps;
+            if (status) {
+                ctx->err = M->conlin ? "CONLIN interior-point loop reached max_newton"
+                                     : "MMA interior-point loop reached max_newton";
+                return PF_NOT_CONVERGED;
+            }
+            if (!M->conlin) {
+                std::swap(M->L, M->alpha);
+                std::swap(M->U, M->beta);
+            }
+            return mma_accept(ctx, xk, f);
+        }
+    }
     const unsigned gg = gsize(n);
     double* part = ctx->red.partials;
     if (M->conlin)
@@ -2880,12 +2947,10 @@ int mma_update_device(pf_ctx* ctx, double* xk, double f, const double* dfdx, dou
         dll += S[0];
         double Dlly = Dl + 1.0 / Dy;
         double dlly = dll + dly / Dy;
-        double A[2][2] = {{0.0 + S[1], a}, {a, -zeta / z}};
-        A[0][0] += Dlly;
-        double B[2] = {dlly - S[2], dlz};
-        double sol[2];
-        solve2(A, B, sol);
-        double dlam = sol[0], dz = sol[1];
+        double A00 = 0.0 + S[1];
+        A00 += Dlly;
+        double dlam, dz;
+        mma_solve2(A00, a, a, -zeta / z, dlly - S[2], dlz, dlam, dz);
         k_mma_newton_b<<<gg, kBlock, 0, ctx->stream>>>(n, dlam, eps, M->x, M->gsi, M->ita, M->alpha, M->beta, M->G,
                                                       M->Dx, M->dlx, M->dx, M->dgsi, M->dita, part);
         PF_TRY(check_launch(ctx));
@@ -2935,15 +3000,8 @@ int mma_update_device(pf_ctx* ctx, double* xk, double f, const double* dfdx, dou
         if (dw1 < 0.9 * eps) eps *= 0.1;
         else eps *= 1.0;
     }
-    M->previousvalue = f;
-    M->k++;
-    const size_t eb = sizeof(double) * n;
-    PF_HIP(hipMemcpyAsync(M->xkm2, M->xkm1, eb, hipMemcpyDeviceToDevice, ctx->stream));
-    PF_HIP(hipMemcpyAsync(M->xkm1, xk, eb, hipMemcpyDeviceToDevice, ctx->stream));
-    PF_HIP(hipMemcpyAsync(xk, M->x, eb, hipMemcpyDeviceToDevice, ctx->stream));
-    PF_TRY(sync(ctx));
     if (steps_out) *steps_out = l;
-    return PF_OK;
+    return mma_accept(ctx, xk, f);
 }
 
 int mma_init_device(pf_ctx* ctx, const pf_mma_params* prm, bool conlin = false) {
@@ -3028,6 +3086,7 @@ int pf_create(pf_ctx** out, int device) {
     if (rc == PF_OK) {
         ctx->res_slots = (u64*)(ctx->red.partials + 8L * kMaxPartials);
         ctx->d_res = (ResDev*)(ctx->res_slots + kResWords);
+        if (hipMemset(ctx->res_slots, 0, kResWords * 8) != hipSuccess) rc = PF_ERR_HIP;  // tags start at 1
     }
     if (rc == PF_OK) rc = dalloc(ctx, &ctx->red.counter, 1);
     if (rc == PF_OK) rc = dalloc(ctx, &ctx->red.out, 16);

@@ -123,26 +123,33 @@ __device__ inline bool res_wait_pair(const u64* p, unsigned tag, Vec2<float>& v)
 
 // Wavefront sum, complete in lane 63 only: row shifts and row broadcasts (DPP)
 // instead of a butterfly through the LDS crossbar, a fixed order of additions.
-template <int CTRL, int ROWS>
-__device__ inline double res_dpp_add(double v) {
+// MAX: the maximum of non-negative values instead.
+template <bool MAX>
+__device__ inline double res_op(double a, double b) {
+    if constexpr (MAX) return (a < b) ? b : a;
+    else return a + b;
+}
+template <bool MAX, int CTRL, int ROWS>
+__device__ inline double res_dpp_op(double v) {
     const u64 b = (u64)__double_as_longlong(v);
     const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, ROWS, 0xf, false);
     const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, ROWS, 0xf, false);
-    return v + res_join(lo, hi);
+    return res_op<MAX>(v, res_join(lo, hi));
 }
+template <bool MAX = false>
 __device__ inline double res_wave_sum(double v) {
-    v = res_dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of a row has its sum
-    v = res_dpp_add<0x112, 0xf>(v);
-    v = res_dpp_add<0x114, 0xf>(v);
-    v = res_dpp_add<0x118, 0xf>(v);
-    v = res_dpp_add<0x142, 0xa>(v);  // lane 15 of rows 0, 2 to rows 1, 3
-    v = res_dpp_add<0x143, 0xc>(v);  // lane 31 to rows 2, 3
+    v = res_dpp_op<MAX, 0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of a row has its sum
+    v = res_dpp_op<MAX, 0x112, 0xf>(v);
+    v = res_dpp_op<MAX, 0x114, 0xf>(v);
+    v = res_dpp_op<MAX, 0x118, 0xf>(v);
+    v = res_dpp_op<MAX, 0x142, 0xa>(v);  // lane 15 of rows 0, 2 to rows 1, 3
+    v = res_dpp_op<MAX, 0x143, 0xc>(v);  // lane 31 to rows 2, 3
     return v;
 }
 
 struct ResLds {
-    double part[3 * 16];  // this workgroup's sums per wave
-    double sum[3 * 4];    // all workgroups' sums per group of 64 slots
+    double part[4 * 16];  // this workgroup's sums per wave
+    double sum[4 * 4];    // all workgroups' sums per group of 64 slots
     int bad;
 };
 
@@ -169,11 +176,11 @@ __device__ inline void res_pause() {
 
 // This workgroup's sums of v, published under `tag` by K*2 threads.  The
 // barrier inside also ends the phase that filled v.
-template <int K, int NT>
+template <int K, int NT, bool MAX = false>
 __device__ inline void res_publish(double (&v)[K], ResLds& L, u64* slots, unsigned tag) {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
 #pragma unroll
-    for (int k = 0; k < K; k++) v[k] = res_wave_sum(v[k]);
+    for (int k = 0; k < K; k++) v[k] = res_wave_sum<MAX>(v[k]);
     if (lane == 63) {
 #pragma unroll
         for (int k = 0; k < K; k++) L.part[k * 16 + w] = v[k];
@@ -182,20 +189,20 @@ __device__ inline void res_publish(double (&v)[K], ResLds& L, u64* slots, unsign
     if (t < 2 * K) {
         double s = 0.0;
 #pragma unroll
-        for (int i = 0; i < NT / 64; i++) s += L.part[(t >> 1) * 16 + i];
+        for (int i = 0; i < NT / 64; i++) s = res_op<MAX>(s, L.part[(t >> 1) * 16 + i]);
         res_put(res_slot(slots, tag, t >> 1, blockIdx.x) + (t & 1), tag, res_half(s, t & 1));
     }
 }
 // All workgroups' sums into v (the same bits in every thread); false: stalled.
 // Threads [NT / 2, NT / 2 + 256) (NT = 256: all) each read one workgroup's slot.
-template <int K, int NT>
+template <int K, int NT, bool MAX = false>
 __device__ inline bool res_collect(double (&v)[K], ResLds& L, const u64* slots, unsigned tag) {
     if (gridDim.x == 1) {  // nobody to wait for
 #pragma unroll
         for (int k = 0; k < K; k++) {
             double s = 0.0;
 #pragma unroll
-            for (int i = 0; i < NT / 64; i++) s += L.part[k * 16 + i];
+            for (int i = 0; i < NT / 64; i++) s = res_op<MAX>(s, L.part[k * 16 + i]);
             v[k] = wave_uniform(s);
         }
         __syncthreads();
@@ -214,7 +221,7 @@ __device__ inline bool res_collect(double (&v)[K], ResLds& L, const u64* slots, 
             for (int k = 0; k < K; k++) s[k] = res_join(q[2 * k], q[2 * k + 1]);
         }
 #pragma unroll
-        for (int k = 0; k < K; k++) s[k] = res_wave_sum(s[k]);
+        for (int k = 0; k < K; k++) s[k] = res_wave_sum<MAX>(s[k]);
         if (lane == 63) {
 #pragma unroll
             for (int k = 0; k < K; k++) L.sum[k * 4 + (t >> 6)] = s[k];
@@ -224,7 +231,8 @@ __device__ inline bool res_collect(double (&v)[K], ResLds& L, const u64* slots, 
     if (L.bad) return false;
 #pragma unroll
     for (int k = 0; k < K; k++)
-        v[k] = wave_uniform(((L.sum[k * 4] + L.sum[k * 4 + 1]) + L.sum[k * 4 + 2]) + L.sum[k * 4 + 3]);
+        v[k] = wave_uniform(res_op<MAX>(
+            res_op<MAX>(res_op<MAX>(L.sum[k * 4], L.sum[k * 4 + 1]), L.sum[k * 4 + 2]), L.sum[k * 4 + 3]));
     return true;
 }
 
