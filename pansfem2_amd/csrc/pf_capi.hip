@@ -269,6 +269,8 @@ void free_grid(pf_ctx* ctx) {
     ctx->have_E = false;
     ctx->have_filter = false;
     ctx->have_lists = false;
+    dfree(ctx->d_fcol);
+    ctx->have_fcol = false;
     release_net(ctx);
 }
 
@@ -2636,21 +2638,82 @@ int solve_nodal(pf_ctx* ctx, int op, const double* b, double* x, double eps, int
 }
 
 // ------------------------------------------------------------------ OC ----
+// The bisection in one resident launch (k_oc_resident), its result in h_oc;
+// *ran is false, and nothing has been done, with the projection in the closure,
+// more elements than the chip's registers hold or a launch that cannot be made
+// or stalled.
+int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const double* x, const double* dfdx,
+                const double* dgdx, double* xplus, bool* ran) {
+    *ran = false;
+    constexpr int NT = kOcResThreads;
+    const long ne = ctx->ne, most = (long)ctx->res_wgs * NT;
+    if (ctx->res_stalled || most <= 0 || ne > 16 * most || prm->beta > 0.0 || max_steps > 1000000) return PF_OK;
+    if (!ctx->have_fcol) {
+        if (!ctx->d_fcol) PF_TRY(dalloc(ctx, &ctx->d_fcol, ne));
+        k_filter_colsum<<<gsize(ne), kBlock, 0, ctx->stream>>>(g3(ctx), ctx->dim, ctx->win, ctx->R, ctx->d_cg, nullptr,
+                                                               xplus);
+        k_filter_colsum<<<gsize(ne), kBlock, 0, ctx->stream>>>(g3(ctx), ctx->dim, ctx->win, ctx->R, ctx->d_cg, xplus,
+                                                               ctx->d_fcol);
+        PF_TRY(check_launch(ctx));
+        ctx->have_fcol = true;
+    }
+    // one element per thread while the workgroups last, then 2, 4, 8, 16
+    int S = 1;
+    while (ne > S * most) S *= 2;
+    const void* kern = S == 1   ? (const void*)k_oc_resident<1>
+                       : S == 2 ? (const void*)k_oc_resident<2>
+                       : S == 4 ? (const void*)k_oc_resident<4>
+                       : S == 8 ? (const void*)k_oc_resident<8>
+                                : (const void*)k_oc_resident<16>;
+    PF_TRY(res_begin(ctx, 0));
+    OcRes A{};
+    A.n = ne;
+    A.max_steps = max_steps;
+    A.tag = ctx->res_tag;
+    ctx->res_tag += (unsigned)max_steps + 1;
+    A.iota = prm->iota; A.move = prm->movelimit; A.leps = prm->lambdaeps;
+    A.vf = prm->vf; A.scale1 = prm->scale1;
+    A.l0 = prm->lambdamin; A.l1 = prm->lambdamax;
+    A.x = x; A.dfdx = dfdx; A.dgdx = dgdx; A.col = ctx->d_fcol; A.xplus = xplus;
+    A.slots = ctx->res_slots;
+    A.R = ctx->d_res;
+    A.O = (OcDev*)ctx->d_oc;
+    void* args[] = {&A};
+    const unsigned wgs = (unsigned)((ne + (long)NT * S - 1) / ((long)NT * S));
+    if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(NT), args, 0, ctx->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return PF_OK;
+    }
+    PF_HIP(hipMemcpyAsync(ctx->h_oc, ctx->d_oc, sizeof(OcDev), hipMemcpyDeviceToHost, ctx->stream));
+    PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
+    PF_TRY(sync(ctx));
+    if (ctx->h_res->stall) {
+        ctx->res_stalled = true;
+        return PF_OK;
+    }
+    *ran = true;
+    return PF_OK;
+}
+
 int oc_device(pf_ctx* ctx, const pf_oc_params* prm, const double* x, const double* dfdx, const double* dgdx,
               double* xplus, double* lambda_out, int* steps_out) {
     PF_CHECK(ctx->have_filter && !ctx->have_lists, PF_ERR_STATE,
              "the device OC closure filters with the grid rule: call pf_filter_setup first");
     OcDev* S = (OcDev*)ctx->d_oc;
-    OcDev init{};
-    init.l0i = prm->lambdamin;
-    init.l1i = prm->lambdamax;
-    PF_HIP(hipMemcpyAsync(S, &init, sizeof(OcDev), hipMemcpyHostToDevice, ctx->stream));
-    PF_HIP(hipMemsetAsync(xplus, 0, sizeof(double) * ctx->ne, ctx->stream));  // xkp1 starts as zeros (OC.h:81)
-    const unsigned g = gsize(ctx->ne);
     const int max_steps = prm->max_steps > 0 ? prm->max_steps : 200;
+    bool resident;
+    PF_TRY(oc_resident(ctx, prm, max_steps, x, dfdx, dgdx, xplus, &resident));
+    if (!resident) {
+        OcDev init{};
+        init.l0i = prm->lambdamin;
+        init.l1i = prm->lambdamax;
+        PF_HIP(hipMemcpyAsync(S, &init, sizeof(OcDev), hipMemcpyHostToDevice, ctx->stream));
+        PF_HIP(hipMemsetAsync(xplus, 0, sizeof(double) * ctx->ne, ctx->stream));  // xkp1 starts as zeros (OC.h:81)
+    }
+    const unsigned g = gsize(ctx->ne);
     const int chunk = 16;
     int k = 0;
-    bool done = false;
+    bool done = resident;
     volatile OcDev* H = (volatile OcDev*)ctx->h_oc;
     // quad4: one launch per bisection step (k_oc_step); hex8: the candidate
     // and the filtered volume in two launches
@@ -2684,12 +2747,12 @@ int oc_device(pf_ctx* ctx, const pf_oc_params* prm, const double* x, const doubl
                                                      S);
         PF_HIP(hipMemcpyAsync((void*)H, S, sizeof(OcDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_TRY(sync(ctx));
-        if (!H->done) {
-            if (lambda_out) *lambda_out = H->lambda_last;
-            if (steps_out) *steps_out = H->steps;
-            ctx->err = "OC bisection did not reach lambdaeps within max_steps";
-            return PF_NOT_CONVERGED;
-        }
+    }
+    if (!H->done) {
+        if (lambda_out) *lambda_out = H->lambda_last;
+        if (steps_out) *steps_out = H->steps;
+        ctx->err = "OC bisection did not reach lambdaeps within max_steps";
+        return PF_NOT_CONVERGED;
     }
     if (lambda_out) *lambda_out = H->lambda_last;
     if (steps_out) *steps_out = H->steps;
@@ -3631,6 +3694,7 @@ int pf_filter_setup(pf_ctx* ctx, double R) {
     ctx->win = (int)std::floor(R / h * (1.0 + 1e-9));
     ctx->have_filter = true;
     ctx->have_lists = false;
+    ctx->have_fcol = false;
     return PF_OK;
 }
 

@@ -110,6 +110,8 @@ struct pf_ctx {
     int win = 0;
     bool have_filter = false;
     bool have_lists = false;
+    double* d_fcol = nullptr;  // column sums of the grid rule's normalised weights, formed when an OC update needs them
+    bool have_fcol = false;
     int32_t *d_fptr = nullptr, *d_fidx = nullptr;
     double* d_fw = nullptr;
 
