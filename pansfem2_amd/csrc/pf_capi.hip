@@ -1010,6 +1010,7 @@ struct MgState {
     int* dof = nullptr;     // their nodal indices
     double* A = nullptr;    // coarsest free-DOF block, inverted in place
     double* W = nullptr;    // inversion scratch
+    double* M = nullptr;    // hex8: the children's contributions to a coarse element (k_mg3_child_matrices), behind W
     std::vector<void*> owned;
 };
 // pixels per workgroup of a weight-gradient launch
@@ -1585,7 +1586,8 @@ int mg_plan(pf_ctx* ctx, int nu, float omega, int prolong) {
     const long nvc = S->L[c].nv;
     PF_TRY(mg_alloc(ctx, &S->dof, nvc));
     PF_TRY(mg_alloc(ctx, &S->A, nvc * nvc));
-    PF_TRY(mg_alloc(ctx, &S->W, nvc * nvc));
+    PF_TRY(mg_alloc(ctx, &S->W, nvc * nvc + (h8 ? 8L * 576 : 0)));
+    S->M = S->W + nvc * nvc;
     return PF_OK;
 }
 
@@ -1606,9 +1608,15 @@ int mg_build(pf_ctx* ctx) {
         MgLevel& a = S->L[l];
         const double* Kf = l == 1 ? nullptr : S->L[l - 1].Ke64;
         if (h8) {
-            const long t = a.ne * 24;
-            k_mg3_coarsen<<<(unsigned)((t + kBlock - 1) / kBlock), kBlock, 0, ctx->stream>>>(
-                a.nx, a.ny, a.nz, ctx->d_E, ctx->d_K0, ctx->d_fix, Kf, a.Ke64, a.Ke32);
+            if (l == 1) {
+                k_mg3_child_matrices<<<18, kBlock, 0, ctx->stream>>>(ctx->d_K0, S->M);
+                k_mg3_coarsen0<<<(unsigned)std::min(a.ne, 4096L), kMg3C0Threads, 0, ctx->stream>>>(
+                    a.nx, a.ny, a.nz, ctx->d_E, ctx->d_K0, S->M, ctx->d_fix, a.Ke64, a.Ke32);
+            } else {
+                const long t = a.ne * 24;
+                k_mg3_coarsen<<<(unsigned)((t + kBlock - 1) / kBlock), kBlock, 0, ctx->stream>>>(a.nx, a.ny, a.nz, Kf,
+                                                                                                 a.Ke64, a.Ke32);
+            }
             k_mg3_diag_full<<<gsize(a.nn), kBlock, 0, ctx->stream>>>(a.nx, a.ny, a.nz, a.Ke64, a.D, a.fix);
         } else {
             const long t = a.ne * 8;
@@ -3190,8 +3198,6 @@ int pf_destroy(pf_ctx* ctx) {
     dfree(ctx->d_K0gf);
     dfree(ctx->d_K0m);
     dfree(ctx->d_K0mf);
-    dfree(ctx->d_K0p);
-    dfree(ctx->d_K0pf);
     dfree(ctx->red.partials);
     dfree(ctx->red.counter);
     dfree(ctx->red.out);
@@ -3317,26 +3323,20 @@ int pf_set_element_matrix(pf_ctx* ctx, const double* K0, int nd) {
         PF_TRY(dalloc(ctx, &ctx->d_K0gf, nd * nd));
         PF_HIP(hipMemcpyAsync(ctx->d_K0g, g64.data(), sizeof(double) * nd * nd, hipMemcpyHostToDevice, ctx->stream));
         PF_HIP(hipMemcpyAsync(ctx->d_K0gf, g32.data(), sizeof(float) * nd * nd, hipMemcpyHostToDevice, ctx->stream));
-        // the MFMA operator's A fragments
-        std::vector<double> m64(768);
-        std::vector<float> m32(768);
-        double par[kH8ParityCoefs];
-        float par32[kH8ParityCoefs];
-        dfree(ctx->d_K0p);
-        dfree(ctx->d_K0pf);
-        if (h8_parity_pack(K0, par)) {
-            for (int i = 0; i < kH8ParityCoefs; i++) par32[i] = (float)par[i];
-            PF_TRY(dalloc(ctx, &ctx->d_K0p, kH8ParityCoefs));
-            PF_TRY(dalloc(ctx, &ctx->d_K0pf, kH8ParityCoefs));
-            PF_HIP(hipMemcpy(ctx->d_K0p, par, sizeof(par), hipMemcpyHostToDevice));
-            PF_HIP(hipMemcpy(ctx->d_K0pf, par32, sizeof(par32), hipMemcpyHostToDevice));
-        }
+        // the MFMA operator's A fragments, then the parity blocks
+        std::vector<double> m64(768 + kH8ParityCoefs, 0.0);
+        std::vector<float> m32(768 + kH8ParityCoefs, 0.f);
         h8m_pack_k0(K0, m64.data());
         h8m_pack_k0(K0, m32.data());
-        PF_TRY(dalloc(ctx, &ctx->d_K0m, 768));
-        PF_TRY(dalloc(ctx, &ctx->d_K0mf, 768));
-        PF_HIP(hipMemcpyAsync(ctx->d_K0m, m64.data(), sizeof(double) * 768, hipMemcpyHostToDevice, ctx->stream));
-        PF_HIP(hipMemcpyAsync(ctx->d_K0mf, m32.data(), sizeof(float) * 768, hipMemcpyHostToDevice, ctx->stream));
+        const bool parity = h8_parity_pack(K0, m64.data() + 768);
+        for (int i = 0; i < kH8ParityCoefs; i++) m32[768 + i] = (float)m64[768 + i];
+        const long nm = (long)m64.size();
+        PF_TRY(dalloc(ctx, &ctx->d_K0m, nm));
+        PF_TRY(dalloc(ctx, &ctx->d_K0mf, nm));
+        PF_HIP(hipMemcpyAsync(ctx->d_K0m, m64.data(), sizeof(double) * nm, hipMemcpyHostToDevice, ctx->stream));
+        PF_HIP(hipMemcpyAsync(ctx->d_K0mf, m32.data(), sizeof(float) * nm, hipMemcpyHostToDevice, ctx->stream));
+        ctx->d_K0p = parity ? ctx->d_K0m + 768 : nullptr;
+        ctx->d_K0pf = parity ? ctx->d_K0mf + 768 : nullptr;
     }
     return sync(ctx);
 }

@@ -68,7 +68,7 @@ struct pf_ctx {
     float* d_K0gf = nullptr;
     double* d_K0m = nullptr;  // hex8: K0 as the MFMA operator's A fragments (h8m_pack_k0)
     float* d_K0mf = nullptr;
-    double* d_K0p = nullptr;  // hex8: K0's parity blocks (h8_parity_pack); null when it has none
+    double* d_K0p = nullptr;  // hex8: K0's parity blocks (h8_parity_pack), behind d_K0m; null when it has none
     float* d_K0pf = nullptr;
 
     // material / design

@@ -585,8 +585,8 @@ __global__ void __launch_bounds__(256) k_filter_colsum(G3 g, int dim, int win, d
 // elements per thread stay in registers.  The filter is linear, so the filtered
 // volume is the column sums' product with x+, the same sum in another order, and
 // a step is S candidates and one exchanged sum.  The launched form filters x+
-// in every step: per step 24 us at 1024x512 (8.6 at 120x40) and 36 at
-// 128x64x64; resident 3.4 (1.9) and 3.4, bound by the exchange.
+// in every step: per step 8.6 us at 120x40 and 36 at 128x64x64; resident 2.3
+// and 2.1, bound by the exchange.
 struct OcRes {
     long n;
     int max_steps;
