@@ -1218,7 +1218,8 @@ void conv_wgrad_t(pf_ctx* ctx, float* wpart, int H, int W, const bf16* X, const 
     const int ppb = kWgradPixels;
     const long npx = (long)H * W;
     const int nb = (int)((npx + ppb - 1) / ppb);
-    k_conv_wgrad_tap<2, CI, CO><<<dim3(nb, 9), 256, 0, ctx->stream>>>(H, W, 1, X, dZ, wpart, ppb);
+    k_conv_wgrad<2, CI, CO><<<dim3(nb, 3, wgrad_tiles(CI, CO)), 64 * wgrad_waves(CI, CO), 0, ctx->stream>>>(
+        H, W, 1, X, dZ, wpart, ppb);
     const int n = 9 * CI * CO;
     k_wgrad_reduce<<<nblocks(n), kBlock, 0, ctx->stream>>>(wpart, nb, n, dW);
 }
@@ -1314,7 +1315,8 @@ void conv3_wgrad_t(pf_ctx* ctx, float* wpart, int H, int W, int Dp, const bf16* 
     const int ppb = kWgradPixels;
     const long npx = (long)H * W * Dp;
     const int nb = (int)((npx + ppb - 1) / ppb);
-    k_conv_wgrad_tap<3, CI, CO><<<dim3(nb, 27), 256, 0, ctx->stream>>>(H, W, Dp, X, dZ, wpart, ppb);
+    k_conv_wgrad<3, CI, CO><<<dim3(nb, 9, wgrad_tiles(CI, CO)), 64 * wgrad_waves(CI, CO), 0, ctx->stream>>>(
+        H, W, Dp, X, dZ, wpart, ppb);
     const int n = 27 * CI * CO;
     k_wgrad_reduce<<<nblocks(n), kBlock, 0, ctx->stream>>>(wpart, nb, n, dW);
 }

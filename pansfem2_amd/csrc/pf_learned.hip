@@ -404,111 +404,173 @@ __global__ void __launch_bounds__(256) k_conv3_fwd_tile(int H, int W, int Dp, co
     }
 }
 
-// The 8 channels of one pixel (v) into 8 channel-major LDS rows of stride rs.
-__device__ inline void st8_cols(bf16* dst, int rs, uint4 v) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int t = 0; t < 8; t++) dst[t * rs] = (bf16)((t & 1) ? (w[t >> 1] >> 16) : (w[t >> 1] & 0xFFFFu));
-}
-
 // -------------------------------------------------------- weight gradient --
 // dW[tap][co][ci] = sum_p dZ[p][co] X[p + off(tap)][ci] (2D: DIM = 2, taps
 // 3 (di + 1) + (dj + 1); 3D: DIM = 3 on H x W x Dp, taps 9 (di + 1) +
 // 3 (dj + 1) + (dk + 1)), FP32 partials per block of ppb pixels (reduced
-// afterwards in a fixed order).  One workgroup per (block, tap): wave w
-// takes the tap's (output block, input block) accumulators w, w + 4, ...
-// The block's dZ and its tap-shifted X are staged in LDS 256 pixels at a
-// time with 16-byte loads (zeros past the block and where the tap's
-// neighbour leaves the grid), channel-major so that a lane's four pixels of
-// one channel are one 8-byte read; each accumulator sums
-// its MFMAs over the block's 16-pixel chunks in pixel order, lane (g, c)
-// holding pixels 4g..4g+3 of a chunk (dZ channel c of its output block as
-// the A operand, X channel c of its input block as B).
+// afterwards in a fixed order).  One workgroup per (block, line offset, tile of
+// channels): it computes the three taps that differ along the contiguous axis from one
+// staged copy of X.  dZ and X (the piece's pixels shifted by the line offset,
+// and one more on each side) go to LDS as they are in memory, 256 pixels at a
+// time, in planes of 16 channels, 32 bytes per pixel; the next piece is on its
+// way in registers meanwhile, and the two LDS buffers alternate, one barrier
+// per piece.  The matrix core wants four pixels of one channel per lane: the
+// transposing LDS read gives them, lane i of a group of 16 pointing at channels
+// 4 (i & 3) .. + 3 of pixel i >> 2 and getting channel i of the four pixels.
+// A neighbour outside the grid is a lane pointing at a pixel of zeros, so a
+// shift by one pixel is an address, and no copy per tap is needed.  Each
+// accumulator sums its MFMAs over the block's 16-pixel chunks in pixel order.
+//
+// Bound by the latency of a block's 16 pieces, whose order is fixed.  At 1025 x 513
+// nodes and below, per launch: 16 -> 16 channels 27.8 us, 32 -> 32 30.5, 16 <-> 32
+// 26, 32 <-> 64 31; one workgroup per tap that transposed its own copies with
+// 2-byte LDS stores took 53.8, 64.8, 56 and 102.  A wave per (16 x 16 pair, tap)
+// and tiles of at most 32 x 32 channels: with the three taps in one wave 32 -> 32
+// took 58.6 and 32 <-> 64 67; with the LDS reads next to their products instead
+// of eight chunks ahead 68.7 and 75.
+constexpr int wgrad_tile(int c) { return c < 32 ? c : 32; }
+constexpr int wgrad_waves(int cin, int cout) { return 3 * (wgrad_tile(cin) / 16) * (wgrad_tile(cout) / 16); }
+constexpr int wgrad_tiles(int cin, int cout) { return (cin / wgrad_tile(cin)) * (cout / wgrad_tile(cout)); }
+
 template <int DIM, int CIN, int COUT>
-__global__ void __launch_bounds__(256) k_conv_wgrad_tap(int H, int W, int Dp, const bf16* __restrict__ X,
-                                                        const bf16* __restrict__ dZ, float* __restrict__ part,
-                                                        int ppb) {
+__global__ void __launch_bounds__(64 * wgrad_waves(CIN, COUT))
+    k_conv_wgrad(int H, int W, int Dp, const bf16* __restrict__ X, const bf16* __restrict__ dZ,
+                 float* __restrict__ part, int ppb) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     constexpr int NTAP = DIM == 3 ? 27 : 9;
-    constexpr int CT = COUT / 16, KT = CIN / 16, NPAIR = CT * KT, NPW = (NPAIR + 3) / 4;
-    constexpr int SP = 256;      // pixels per staged piece
-    constexpr int RS = SP + 4;   // LDS row stride: channel-major rows, 8 bytes apart in banks
-    __shared__ __align__(16) bf16 sZ[COUT * RS];
-    __shared__ __align__(16) bf16 sX[CIN * RS];
-    const int tap = blockIdx.y;
-    const int di = DIM == 3 ? tap / 9 - 1 : tap / 3 - 1;
-    const int dj = DIM == 3 ? (tap / 3) % 3 - 1 : tap % 3 - 1;
-    const int dk = DIM == 3 ? tap % 3 - 1 : 0;
-    const long plane = DIM == 3 ? (long)W * Dp : (long)W;  // pixels per i
-    const int D = DIM == 3 ? Dp : 1;
-    const long npx = (long)H * plane;
-    const long off = (long)di * plane + (long)dj * D + dk;
+    constexpr int TI = wgrad_tile(CIN), TO = wgrad_tile(COUT);  // the workgroup's channels
+    constexpr int CT = TO / 16, KT = TI / 16;
+    constexpr int NT = 64 * wgrad_waves(CIN, COUT);
+    constexpr int SP = 256;                            // pixels per piece
+    constexpr int XP = SP + 2, XS = XP + 1;            // staged pixels of X, and the pixel of zeros
+    constexpr int NZ = SP * TO / 8, NX = XP * TI / 8;  // 16-byte chunks
+    constexpr int RZ = (NZ + NT - 1) / NT, RX = (NX + NT - 1) / NT;
+    constexpr int BZ = CT * SP * 16, BX = KT * XS * 16;
+    __shared__ __align__(16) bf16 sm[2 * (BZ + BX)];
+    const int outer = blockIdx.y;  // the tap's offset along all but the contiguous axis
+    const int di = DIM == 3 ? outer / 3 - 1 : outer - 1;
+    const int dj = DIM == 3 ? outer % 3 - 1 : 0;
+    const int D = DIM == 3 ? Dp : W;         // pixels of a line
+    const int L = DIM == 3 ? W : 1;          // lines per i
+    const long npx = (long)H * L * D;
+    const long off = ((long)di * L + dj) * D;
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c16 = l & 15;
+    const int pair = wave / 3, tap = wave - 3 * pair, d = tap - 1;
+    const int ct = pair / KT, kt = pair - ct * KT;
+    const int ti = (int)blockIdx.z % (CIN / TI) * TI, to = (int)blockIdx.z / (CIN / TI) * TO;
     const long p_begin = (long)blockIdx.x * ppb;
-    const long p_end = min(npx, p_begin + ppb);
-    f32x4 acc[NPW];
+    const long p_end = p_begin + ppb < npx ? p_begin + ppb : npx;
+    for (int e = threadIdx.x; e < 2 * KT * 16; e += NT)
+        sm[(e / (KT * 16)) * (BZ + BX) + BZ + ((e / 16) % KT) * XS * 16 + XP * 16 + e % 16] = 0;
+    u32x4 rz[RZ], rx[RX];
+    // pixels outside the tensor are read at its nearest pixel: dZ's are zeroed when
+    // they are staged, X's belong to taps that point at the zeros
+    auto fetch = [&](long s0) {
 #pragma unroll
-    for (int q = 0; q < NPW; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long s0 = p_begin; s0 < p_end; s0 += SP) {
-        __syncthreads();  // the previous piece has been read
-        for (int e = threadIdx.x; e < SP * COUT / 8; e += 256) {
-            const int px = e / (COUT / 8), ch = e - px * (COUT / 8);
-            const long p = s0 + px;
-            uint4 v = {0u, 0u, 0u, 0u};
-            if (p < p_end) v = *reinterpret_cast<const uint4*>(dZ + p * COUT + ch * 8);
-            st8_cols(sZ + ch * 8 * RS + px, RS, v);
+        for (int u = 0; u < RZ; u++) {
+            const int e = threadIdx.x + NT * u, px = e / (TO / 8), ch = e - px * (TO / 8);
+            const long p = s0 + px < npx ? s0 + px : npx - 1;
+            rz[u] = *reinterpret_cast<const u32x4*>(dZ + p * COUT + to + ch * 8);
         }
-        // X at the tap neighbour of each pixel, zero where the neighbour leaves
-        // the grid (or the pixel the block); the division runs once per staged
-        // 16-byte chunk, not per product
-        for (int e = threadIdx.x; e < SP * CIN / 8; e += 256) {
-            const int px = e / (CIN / 8), ch = e - px * (CIN / 8);
-            const int p = (int)(s0 + px);
-            uint4 v = {0u, 0u, 0u, 0u};
-            if (p < p_end) {
-                const int pi = p / (int)plane, r2 = p - pi * (int)plane;
-                const int pj = r2 / D, pk = r2 - pj * D;
-                const int ii = pi + di, jj = pj + dj, kk = pk + dk;
-                if (ii >= 0 && ii < H && jj >= 0 && jj < W && kk >= 0 && kk < D)
-                    v = *reinterpret_cast<const uint4*>(X + (p + off) * CIN + ch * 8);
-            }
-            st8_cols(sX + ch * 8 * RS + px, RS, v);
-        }
-        __syncthreads();
-        for (int c = 0; c < SP / 16; c++) {
-            const long p0 = s0 + 16 * c;
-            if (p0 >= p_end) break;
-            // the lane's four pixels are 4g .. 4g + 3 of the chunk; pixels past
-            // the block and neighbours outside the grid are zeros in LDS
-            const int lp = 16 * c + 4 * g;  // the lane's first pixel in the piece
 #pragma unroll
-            for (int q = 0; q < NPW; q++) {
-                const int pr = wave + 4 * q;
-                if (pr >= NPAIR) break;
-                const int ct = pr / KT, kt = pr - ct * KT;
-                const bf16x4 a = *reinterpret_cast<const bf16x4*>(sZ + (ct * 16 + c16) * RS + lp);
-                const bf16x4 b = *reinterpret_cast<const bf16x4*>(sX + (kt * 16 + c16) * RS + lp);
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[q], 0, 0, 0);
+        for (int u = 0; u < RX; u++) {
+            const int e = threadIdx.x + NT * u, px = e / (TI / 8), ch = e - px * (TI / 8);
+            long p = s0 + off - 1 + px;
+            p = p < 0 ? 0 : p < npx ? p : npx - 1;
+            rx[u] = *reinterpret_cast<const u32x4*>(X + p * CIN + ti + ch * 8);
+        }
+    };
+    auto stage = [&](long s0, bf16* buf) {
+#pragma unroll
+        for (int u = 0; u < RZ; u++) {
+            const int e = threadIdx.x + NT * u, px = e / (TO / 8), ch = e - px * (TO / 8);
+            if (NZ % NT == 0 || e < NZ)
+                *reinterpret_cast<u32x4*>(buf + ((ch >> 1) * SP + px) * 16 + (ch & 1) * 8) =
+                    s0 + px < p_end ? rz[u] : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int u = 0; u < RX; u++) {
+            const int e = threadIdx.x + NT * u, px = e / (TI / 8), ch = e - px * (TI / 8);
+            if (NX % NT == 0 || e < NX)
+                *reinterpret_cast<u32x4*>(buf + BZ + ((ch >> 1) * XS + px) * 16 + (ch & 1) * 8) = rx[u];
+        }
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // the pixel this lane points at, 4 g + (c16 >> 2) of each chunk: its place on the
+    // grid, advanced by 16 pixels per chunk
+    const int lp = 4 * g + (c16 >> 2);
+    int left = (int)(p_end - p_begin) - lp;  // pixels of the block from here on
+    int pi, pj, pk;
+    {
+        const long p = p_begin + lp, line = p / D;
+        pk = (int)(p - line * D);
+        pi = (int)(line / L);
+        pj = (int)(line - (long)pi * L);
+    }
+    const int sk = 16 % D, sj = (16 / D) % L, si = (16 / D) / L;
+    fetch(p_begin);
+    int b = 0;
+    for (long s0 = p_begin; s0 < p_end; s0 += SP, b ^= 1) {
+        bf16* buf = sm + b * (BZ + BX);
+        stage(s0, buf);
+        __syncthreads();  // staged; and every wave has read the piece before the last one
+        if (s0 + SP < p_end) fetch(s0 + SP);
+        const bf16* z = buf + ct * SP * 16 + lp * 16 + 4 * (c16 & 3);
+        const bf16* x = buf + BZ + kt * XS * 16 + 4 * (c16 & 3);
+        // whole pieces (chunks past the block add zeros), eight chunks at a time: their
+        // LDS reads are all issued before their products
+        for (int c0 = 0; c0 < SP / 16; c0 += 8) {
+            bf16x4 a[8], v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int c = c0 + u;
+                const bool in = (left > 0) & ((unsigned)(pi + di) < (unsigned)H) &
+                                (DIM == 2 || (unsigned)(pj + dj) < (unsigned)W);
+                a[u] = __builtin_bit_cast(bf16x4,
+                                          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(z + c * 256)));
+                const int px = (in & ((unsigned)(pk + d) < (unsigned)D)) ? 16 * c + lp + tap : XP;
+                v[u] = __builtin_bit_cast(bf16x4,
+                                          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(x + px * 16)));
+                left -= 16;
+                pk += sk;
+                const int cy = pk >= D;
+                pk -= cy ? D : 0;
+                if (DIM == 2) {
+                    pi += si + cy;
+                } else {
+                    pj += sj + cy;
+                    const int cj = pj >= W;
+                    pj -= cj ? W : 0;
+                    pi += si + cj;
+                }
             }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[u], v[u], acc, 0, 0, 0);
         }
     }
     float* out = part + (long)blockIdx.x * NTAP * COUT * CIN;
 #pragma unroll
-    for (int q = 0; q < NPW; q++) {
-        const int pr = wave + 4 * q;
-        if (pr >= NPAIR) break;
-        const int ct = pr / KT, kt = pr - ct * KT;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int cor = ct * 16 + 4 * g + t;
-            out[((long)tap * COUT + cor) * CIN + kt * 16 + c16] = acc[q][t];
-        }
-    }
+    for (int t = 0; t < 4; t++)
+        out[((long)(3 * outer + tap) * COUT + to + ct * 16 + 4 * g + t) * CIN + ti + kt * 16 + c16] = acc[t];
 }
 
+// The blocks' partials in block order, 16 loads in flight (4.8 us a layer; 14.6
+// one by one).
 __global__ void k_wgrad_reduce(const float* __restrict__ part, int nparts, int n, float* __restrict__ dW) {
     for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
         float s = 0.f;
-        for (int b = 0; b < nparts; b++) s += part[(long)b * n + q];
+        int b = 0;
+        for (; b + 16 <= nparts; b += 16) {
+            float v[16];
+#pragma unroll
+            for (int t = 0; t < 16; t++) v[t] = part[(long)(b + t) * n + q];
+#pragma unroll
+            for (int t = 0; t < 16; t++) s += v[t];
+        }
+        for (; b < nparts; b++) s += part[(long)b * n + q];
         dW[q] = s;
     }
 }

@@ -86,3 +86,19 @@ def test_conv_raw_rejects_unsupported_channels(ctx):
     import pansfem2_amd as pa
     with pytest.raises(pa.PfError):
         ctx.conv_raw(np.zeros((4, 4, 8), np.float32), np.zeros((9, 16, 8), np.float32))
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (40, 3), (1, 5000), (4097, 1), (300, 17), (1, 1, 37), (30, 2, 3), (3, 40, 1),
+                                   (20, 20, 20)])
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 32), (32, 16), (32, 32), (64, 32)])
+def test_conv_weight_gradient_line_edges_exact(ctx, cin, cout, shape):
+    """Lines shorter than a 16-pixel chunk (a lane's pixel crosses several
+    lines, in 3D several planes, from one chunk to the next), one line of more
+    than a block of 4096 pixels, and blocks that end inside a chunk."""
+    rng = np.random.default_rng(400 + cin + cout + shape[0])
+    x = ints(rng, shape + (cin,), -2, 2)
+    dz = ints(rng, shape + (cout,), -2, 2)
+    g = ctx.conv_wgrad_raw(x, dz)
+    _, ref = cn.conv_grads(x.astype(np.float64), dz.astype(np.float64), np.zeros((3 ** len(shape), cout, cin)))
+    assert np.sum(np.abs(x)) * 2 < 2 ** 24
+    assert np.array_equal(g.astype(np.float64), ref), float(np.max(np.abs(g - ref)))
