@@ -1069,7 +1069,6 @@ struct LearnedNet {
 
 namespace {
 
-const int kNetLayers = 12;
 int moduli_from_rho(pf_ctx* ctx);
 
 long lvl_px(LearnedNet* N, int lv) { return (long)N->H[lv] * N->Wd[lv] * N->Dz[lv]; }
@@ -1427,54 +1426,40 @@ int net_backward(pf_ctx* ctx) {
         return PF_OK;
     };
     auto relu_bwd = [&](int lv, int C, const bf16* Y, bf16* g) {
-        long n = lvl_px(N, lv) * C;
-        k_relu_bwd<<<gsize(n), kBlock, 0, ctx->stream>>>(n, Y, g);
+        const long n8 = lvl_px(N, lv) * C / 8;
+        k_relu_bwd<<<gsize(n8), kBlock, 0, ctx->stream>>>(n8, (const uint4*)Y, (uint4*)g);
     };
-    auto up_bwd = [&](int lv, int C, const bf16* gfine, bf16* gcoarse) {
-        long n = lvl_px(N, lv + 1) * C;
-        if (d3)
-            k_up3_bwd<<<gsize(n), kBlock, 0, ctx->stream>>>(N->H[lv], N->Wd[lv], N->Dz[lv], C, gfine, gcoarse);
-        else
-            k_up2_bwd<<<gsize(n), kBlock, 0, ctx->stream>>>(N->H[lv], N->Wd[lv], C, gfine, gcoarse);
+    auto depth = [&](int lv) { return d3 ? N->Dz[lv] : 1; };
+    // gradient of the decoder output Y on level lv + 1 (C channels) from that of its upsampled sum on level lv
+    auto up_bwd = [&](int lv, int C, const bf16* gfine, const bf16* Y, bf16* g) {
+        k_up_bwd<<<gsize(lvl_px(N, lv + 1) * C / 8), kBlock, 0, ctx->stream>>>(N->H[lv], N->Wd[lv], depth(lv), C, gfine,
+                                                                             Y, g);
     };
-    auto pool_bwd_add = [&](int lv, int C, const bf16* gcoarse, bf16* gfine) {
-        long n = lvl_px(N, lv) * C;
-        if (d3)
-            k_pool3_bwd_add<<<gsize(n), kBlock, 0, ctx->stream>>>(N->H[lv], N->Wd[lv], N->Dz[lv], C, gcoarse, gfine);
-        else
-            k_pool2_bwd_add<<<gsize(n), kBlock, 0, ctx->stream>>>(N->H[lv], N->Wd[lv], C, gcoarse, gfine);
+    // gradient of the encoder output Y on level lv from its skip and pooled branches
+    auto skip_pool_bwd = [&](int lv, int C, const bf16* gskip, const bf16* gcoarse, const bf16* Y, bf16* g) {
+        k_skip_pool_bwd<<<gsize(lvl_px(N, lv) * C / 8), kBlock, 0, ctx->stream>>>(N->H[lv], N->Wd[lv], depth(lv), C,
+                                                                                gskip, gcoarse, Y, g);
     };
-    auto copy = [&](long n, const bf16* a, bf16* b) { k_copy_bf16<<<gsize(n), kBlock, 0, ctx->stream>>>(n, a, b); };
-    const long p0 = lvl_px(N, 0), p1 = lvl_px(N, 1), p2 = lvl_px(N, 2);
     PF_TRY(back(11, N->d0, N->gy, N->gd0));
     relu_bwd(0, 16, N->d0, N->gd0);
     PF_TRY(back(10, N->u0, N->gd0, N->gu0));
-    up_bwd(0, 16, N->gu0, N->gd1);
-    copy(p0 * 16, N->gu0, N->ge0);  // skip branch of u0 = up(d1) + e0
-    relu_bwd(1, 16, N->d1, N->gd1);
+    up_bwd(0, 16, N->gu0, N->d1, N->gd1);
     PF_TRY(back(9, N->u1, N->gd1, N->gu1));
-    up_bwd(1, 32, N->gu1, N->gd2);
-    copy(p1 * 32, N->gu1, N->ge1);
-    relu_bwd(2, 32, N->d2, N->gd2);
+    up_bwd(1, 32, N->gu1, N->d2, N->gd2);
     PF_TRY(back(8, N->u2, N->gd2, N->gu2));
-    up_bwd(2, 32, N->gu2, N->gb3);
-    copy(p2 * 32, N->gu2, N->ge2);
-    relu_bwd(3, 32, N->b3, N->gb3);
+    up_bwd(2, 32, N->gu2, N->b3, N->gb3);
     PF_TRY(back(7, N->a3, N->gb3, N->ga3));
     relu_bwd(3, 64, N->a3, N->ga3);
     PF_TRY(back(6, N->x3, N->ga3, N->gx3));
-    pool_bwd_add(2, 32, N->gx3, N->ge2);
-    relu_bwd(2, 32, N->e2, N->ge2);
+    skip_pool_bwd(2, 32, N->gu2, N->gx3, N->e2, N->ge2);
     PF_TRY(back(5, N->a2, N->ge2, N->ga2));
     relu_bwd(2, 32, N->a2, N->ga2);
     PF_TRY(back(4, N->x2, N->ga2, N->gx2));
-    pool_bwd_add(1, 32, N->gx2, N->ge1);
-    relu_bwd(1, 32, N->e1, N->ge1);
+    skip_pool_bwd(1, 32, N->gu1, N->gx2, N->e1, N->ge1);
     PF_TRY(back(3, N->a1, N->ge1, N->ga1));
     relu_bwd(1, 32, N->a1, N->ga1);
     PF_TRY(back(2, N->x1, N->ga1, N->gx1));
-    pool_bwd_add(0, 16, N->gx1, N->ge0);
-    relu_bwd(0, 16, N->e0, N->ge0);
+    skip_pool_bwd(0, 16, N->gu0, N->gx1, N->e0, N->ge0);
     PF_TRY(back(1, N->a0, N->ge0, N->ga0));
     relu_bwd(0, 16, N->a0, N->ga0);
     PF_TRY(back(0, N->x0, N->ga0, nullptr));
@@ -2374,10 +2359,14 @@ int net_train_step(pf_ctx* ctx, int s, float lr, double* loss) {
     N->adam_t++;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - std::pow(b1, (float)N->adam_t), c2 = 1.f - std::pow(b2, (float)N->adam_t);
-    for (NetLayer& l : N->L)
-        k_adam<<<nblocks(l.size()), kBlock, 0, ctx->stream>>>((int)l.size(), l.W, l.m, l.v, l.g, lr, b1, b2, 1e-8f,
-                                                             c1, c2, 1.0f);
-    PF_TRY(net_refresh_bf16(ctx, N));
+    AdamLayers P;
+    long most = 0;
+    for (int i = 0; i < kNetLayers; i++) {
+        NetLayer& l = N->L[i];
+        P.l[i] = {l.W, l.m, l.v, l.g, l.Wb, l.Wtb, l.ntap, l.cout, l.cin};
+        most = std::max(most, l.size());
+    }
+    k_adam<<<dim3(nblocks(most), kNetLayers), kBlock, 0, ctx->stream>>>(P, lr, b1, b2, 1e-8f, c1, c2);
     return check_launch(ctx);
 }
 
