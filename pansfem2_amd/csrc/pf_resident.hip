@@ -274,7 +274,11 @@ __global__ void __launch_bounds__(NT) k_pcg_q4_resident(ResArgs<T> A) {
     const unsigned nn = (unsigned)(nx + 1) * (ny + 1);
 
     if (t == 0) L.bad = 0;
-    if (A.S->done || A.R->stall) return;
+    // a workgroup that starts after another has given up; S->done is no reason
+    // to leave (the host launches no more once it is set): workgroup 0 sets it
+    // without an exchange when a launch finds its first iterate converged, and
+    // the workgroups that start later have their part of x still to write
+    if (A.R->stall) return;
     for (int h = t; h < (rows + 2) * ss; h += NT) su[h] = Vec2<T>{0, 0};
     for (int h = t; h < (rows + 1) * es; h += NT) {
         const int a = h / es, ei = i0 - 1 + a, ej = j0 - 1 + (h - a * es);

@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(kRes3Threads) k_pcg_h8_resident(Res3Args<T> A)
     T* sq = sp + NT * SL;     // q likewise
 
     if (t == 0) L.bad = 0;
-    if (A.S->done || A.R->stall) return;
+    if (A.R->stall) return;  // S->done is not tested: see k_pcg_q4_resident
 
     // this thread's node values v = t + NT s (component-major); own: counted
     // and written here, fixm: fixed.  Values beyond NV are zeros that take part

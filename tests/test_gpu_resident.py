@@ -97,6 +97,32 @@ def test_zero_load_zero_steps_and_grid_change(pa):
     ctx.close()
 
 
+@pytest.mark.parametrize("form,last", [(0, 2048), (2, 2047)])
+def test_solve_that_ends_with_a_launch(pa, form, last):
+    """A solve whose last iterate is the last that its first launch finishes: the
+    second launch finds it converged before its first exchange, so that every
+    workgroup leaves it by itself, with x complete.  eps is set a billionth above
+    the residual of that iterate; right-hand sides whose earlier residuals
+    already lie below it are passed over."""
+    ctx, _ = problem(pa, 120, 40)
+    ctx.set_pcg_form(form)
+    ctx.assemble_csr()
+    ended = 0
+    for seed in range(60):
+        b = ctx.load() + np.random.default_rng(seed).uniform(-1e-3, 1e-3, ctx.N)
+        _, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=0.0, itrmax=last)
+        x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=st["rel_residual"] * (1.0 + 1e-9))
+        assert st["status"] == 1 and st["iterations"] <= last
+        if st["iterations"] == last:
+            xr, _ = ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-12)
+            assert rel(x, xr) < 1e-7, rel(x, xr)
+            ended += 1
+        if ended == 3:
+            break
+    assert ended == 3, ended
+    ctx.close()
+
+
 def test_fp32_inner_solves(pa):
     """The FP32 variant inside FP64 refinement."""
     ctx, b = problem(pa, 75, 31)

@@ -69,6 +69,31 @@ def test_more_iterations_than_one_launch(pa):
     ctx.close()
 
 
+def test_solve_that_ends_with_a_launch(pa):
+    """A solve whose last iterate is the last of its first launch (2048): the
+    second launch finds it converged before its first exchange, so that every
+    workgroup leaves it by itself, and each has to write its part of x.  eps is
+    set a billionth above the residual of iterate 2048; right-hand sides whose
+    earlier residuals already lie below that are passed over."""
+    ctx, _ = problem(pa, 60, 6, 5)
+    ctx.set_density(np.random.default_rng(3).uniform(0.05, 1.0, 60 * 6 * 5))
+    ctx.assemble_csr()
+    ended = 0
+    for seed in range(60):
+        b = ctx.load() + np.random.default_rng(seed).uniform(-1e-3, 1e-3, ctx.N)
+        _, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=0.0, itrmax=2048)
+        x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=st["rel_residual"] * (1.0 + 1e-9))
+        assert st["status"] == 1 and st["iterations"] <= 2048
+        if st["iterations"] == 2048:
+            xr, _ = ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-12)
+            assert rel(x, xr) < 1e-7, rel(x, xr)
+            ended += 1
+        if ended == 3:
+            break
+    assert ended == 3, ended
+    ctx.close()
+
+
 def test_element_matrix_without_parity_blocks(pa):
     """A matrix that the mirrors do not leave as it is (a sheared material), one
     that is not symmetric and one that resists translations take the general
