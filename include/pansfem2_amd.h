@@ -209,6 +209,24 @@ enum {
     PF_PCG_SINGLE_REDUCTION_RECOMPUTED = 3
 };
 int pf_set_pcg_form(pf_ctx* ctx, int form);
+/* Jacobi-PCG solves with the matrix-free operators, MMA and CONLIN updates and
+ * OC bisections without projection run in one resident kernel where the grid
+ * fits the chip, and in kernels launched per iteration (per Newton or bisection
+ * step) otherwise: on larger grids, where a cooperative launch is refused, and
+ * after a resident kernel's workgroups have waited two seconds for one
+ * another (a stall; the call then starts over).  Until changed:
+ *   PF_RESIDENT_AUTO: so (the default);
+ *   PF_RESIDENT_OFF: always launched;
+ *   PF_RESIDENT_STALL: as AUTO, but a resident solve's launches (2048
+ *     iterations each; an update or bisection is one launch) after the first
+ *     `after` end as stalled, as beside a program that keeps the GPU busy: for
+ *     tests of what follows.
+ * `after` is not used by the other modes.  Has no counterpart in the reference. */
+enum { PF_RESIDENT_AUTO = 0, PF_RESIDENT_OFF = 1, PF_RESIDENT_STALL = 2 };
+int pf_set_resident(pf_ctx* ctx, int mode, int after);
+/* How many solves (inner solves of a mixed one each), updates and bisections
+ * of this context have run resident to their end, and how many have stalled. */
+int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled);
 /* Kernel of the hex8 matrix-free operator inside the fused PCG iteration
  * (pf_pcg, pf_pcg_dev, pf_simp_run and the multigrid PCG's outer FP64
  * operator on hex8 grids), until changed.  Both apply the same operator as

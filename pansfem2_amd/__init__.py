@@ -21,6 +21,7 @@ PF_PCG_SINGLE_REDUCTION_CARRIED, PF_PCG_SINGLE_REDUCTION_RECOMPUTED = 2, 3
 PF_MG_PROLONG_BILINEAR, PF_MG_PROLONG_STIFFNESS = 0, 1
 PF_MG_RESIDUAL_AUTO, PF_MG_RESIDUAL_NODE, PF_MG_RESIDUAL_ELEMENT = 0, 1, 2
 PF_H8_OP_VALU, PF_H8_OP_MFMA = 0, 1
+PF_RESIDENT_AUTO, PF_RESIDENT_OFF, PF_RESIDENT_STALL = 0, 1, 2
 
 _i32p = np.ctypeslib.ndpointer(np.int32, flags="C_CONTIGUOUS")
 _f64p = np.ctypeslib.ndpointer(np.float64, flags="C_CONTIGUOUS")
@@ -106,6 +107,8 @@ def lib():
             "pf_pcg": ([c_void_p, c_int, _f64p, _f64p, c_double, c_int, P(SolveStats)], c_int),
             "pf_pcg_dev": ([c_void_p, c_int, c_void_p, c_void_p, c_double, c_int, P(SolveStats)], c_int),
             "pf_set_pcg_form": ([c_void_p, c_int], c_int),
+            "pf_set_resident": ([c_void_p, c_int, c_int], c_int),
+            "pf_resident_runs": ([c_void_p, P(c_int64), P(c_int64)], c_int),
             "pf_set_h8_operator": ([c_void_p, c_int], c_int),
             "pf_mg_setup": ([c_void_p, c_int, c_double], c_int),
             "pf_mg_set_prolongation": ([c_void_p, c_int], c_int),
@@ -350,6 +353,20 @@ class Context:
         recomputed on a two-node halo) or PF_PCG_SINGLE_REDUCTION (the
         carried kernel while its working set stays below 150 MB)."""
         self._ck(lib().pf_set_pcg_form(self._h, form))
+
+    def set_resident(self, mode, after=0):
+        """PF_RESIDENT_AUTO (the default: one resident kernel per solve, MMA /
+        CONLIN update and OC bisection where the grid fits the chip),
+        PF_RESIDENT_OFF (always the launched kernels) or PF_RESIDENT_STALL
+        (resident launches after the first `after` of a solve end as stalled:
+        for tests of the fallback)."""
+        self._ck(lib().pf_set_resident(self._h, mode, after))
+
+    def resident_runs(self):
+        """(ended, stalled): resident solves, updates and bisections so far."""
+        d, s = ctypes.c_int64(0), ctypes.c_int64(0)
+        self._ck(lib().pf_resident_runs(self._h, ctypes.byref(d), ctypes.byref(s)))
+        return d.value, s.value
 
     def set_h8_operator(self, kind):
         """PF_H8_OP_VALU (one node per thread on the vector units) or

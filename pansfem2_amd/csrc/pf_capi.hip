@@ -476,6 +476,22 @@ const void* res_kernel(const ResShape& sh) {
     return nullptr;
 }
 
+// whether this context's solves and updates may run resident
+bool res_on(const pf_ctx* ctx) {
+    return ctx->res_wgs >= 1 && ctx->res_mode != PF_RESIDENT_OFF && !ctx->res_stalled;
+}
+// Before launch number `launch` of a resident solve: PF_RESIDENT_STALL's flag.
+void res_force(pf_ctx* ctx, int launch) {
+    if (ctx->res_mode == PF_RESIDENT_STALL && launch >= ctx->res_after) k_res_stall<<<1, 1, 0, ctx->stream>>>(ctx->d_res);
+}
+// After a resident launch (h_res copied back): whether a workgroup gave up.
+bool res_gave_up(pf_ctx* ctx) {
+    if (!ctx->h_res->stall) return false;
+    ctx->res_stalled = true;
+    ctx->res_stalls++;
+    return true;
+}
+
 constexpr int kResChunk = 2048;  // iterations per launch: other streams get the GPU in between
 
 // Exchange buffer of `words` words for a solve that starts now, and the
@@ -507,7 +523,9 @@ int res_run(pf_ctx* ctx, const void* kern, int wgs, int nt, size_t lds, ARGS& A,
     A.R = ctx->d_res;
     A.fix = ctx->d_fix;
     const PcgDev* H = (const PcgDev*)ctx->h_pcg;
+    int launch = 0;
     for (long m = 0;;) {
+        res_force(ctx, launch++);
         A.m0 = (int)m;
         A.m1 = (int)std::min(end, m + kResChunk);
         A.last = A.m1 == end;
@@ -523,14 +541,12 @@ int res_run(pf_ctx* ctx, const void* kern, int wgs, int nt, size_t lds, ARGS& A,
         PF_HIP(hipMemcpyAsync(ctx->h_pcg, A.S, sizeof(PcgDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_TRY(sync(ctx));
-        if (ctx->h_res->stall) {
-            ctx->res_stalled = true;
-            return PF_OK;
-        }
+        if (res_gave_up(ctx)) return PF_OK;
         m = A.m1;
         if (H->done || m >= end) break;
     }
     *ran = true;
+    ctx->res_done++;
     out.iterations = H->iterations;
     out.status = H->status;
     out.rnorm = H->rnorm;
@@ -552,7 +568,7 @@ template <class T>
 int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s, T* p, T* w, double eps, int itrmax,
                  PcgRun& out, bool* ran) {
     *ran = false;
-    if (ctx->res_wgs < 1 || ctx->res_stalled) return PF_OK;
+    if (!res_on(ctx)) return PF_OK;
     const ResShape sh = res_pick<T>(ctx);
     if (!sh.gi) return PF_OK;
     const void* kern = sr ? res_kernel<T, true>(sh) : res_kernel<T, false>(sh);
@@ -618,7 +634,7 @@ Res3Shape res3_pick(const pf_ctx* ctx) {
 }
 
 bool res3_applies(const pf_ctx* ctx) {
-    return ctx->res_wgs >= 1 && !ctx->res_stalled && ctx->d_K0p && ctx->h8_op < 0;
+    return res_on(ctx) && ctx->d_K0p && ctx->h8_op < 0;
 }
 
 // The same for hex8 (k_pcg_h8_resident), ScalingCG's order; only for an
@@ -2697,7 +2713,7 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     *ran = false;
     constexpr int NT = kOcResThreads;
     const long ne = ctx->ne, most = (long)ctx->res_wgs * NT;
-    if (ctx->res_stalled || most <= 0 || ne > 16 * most || prm->beta > 0.0 || max_steps > 1000000) return PF_OK;
+    if (!res_on(ctx) || ne > 16 * most || prm->beta > 0.0 || max_steps > 1000000) return PF_OK;
     if (!ctx->have_fcol) {
         if (!ctx->d_fcol) PF_TRY(dalloc(ctx, &ctx->d_fcol, ne));
         k_filter_colsum<<<gsize(ne), kBlock, 0, ctx->stream>>>(g3(ctx), ctx->dim, ctx->win, ctx->R, ctx->d_cg, nullptr,
@@ -2728,6 +2744,7 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     A.slots = ctx->res_slots;
     A.R = ctx->d_res;
     A.O = (OcDev*)ctx->d_oc;
+    res_force(ctx, 0);
     void* args[] = {&A};
     const unsigned wgs = (unsigned)((ne + (long)NT * S - 1) / ((long)NT * S));
     if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(NT), args, 0, ctx->stream) != hipSuccess) {
@@ -2737,10 +2754,8 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     PF_HIP(hipMemcpyAsync(ctx->h_oc, ctx->d_oc, sizeof(OcDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_TRY(sync(ctx));
-    if (ctx->h_res->stall) {
-        ctx->res_stalled = true;
-        return PF_OK;
-    }
+    if (res_gave_up(ctx)) return PF_OK;
+    ctx->res_done++;
     *ran = true;
     return PF_OK;
 }
@@ -2924,7 +2939,7 @@ int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, c
     const int max_newton = P.max_newton > 0 ? P.max_newton : 500;
     constexpr int NT = kMmaResThreads;
     const long most = (long)ctx->res_wgs * NT;
-    if (ctx->res_stalled || most <= 0 || M->n > 4 * most || max_newton > 100000) return PF_OK;
+    if (!res_on(ctx) || M->n > 4 * most || max_newton > 100000) return PF_OK;
     // one variable per thread while the workgroups last, then two, then four
     const int S = M->n <= most ? 1 : M->n <= 2 * most ? 2 : 4;
     const void* kern = M->conlin ? (S == 1 ? (const void*)k_mma_resident<1, true>
@@ -2949,6 +2964,7 @@ int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, c
     A.xo = M->x; A.Lo = M->alpha; A.Uo = M->beta;
     A.slots = ctx->res_slots;
     A.R = ctx->d_res;
+    res_force(ctx, 0);
     void* args[] = {&A};
     const unsigned wgs = (unsigned)((M->n + (long)NT * S - 1) / ((long)NT * S));
     if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(NT), args, 0, ctx->stream) != hipSuccess) {
@@ -2957,10 +2973,8 @@ int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, c
     }
     PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_TRY(sync(ctx));
-    if (ctx->h_res->stall) {
-        ctx->res_stalled = true;
-        return PF_OK;
-    }
+    if (res_gave_up(ctx)) return PF_OK;
+    ctx->res_done++;
     *steps = (int)ctx->h_res->v[0];
     *status = (int)ctx->h_res->v[1];
     *ran = true;
@@ -3657,6 +3671,23 @@ int pf_set_pcg_form(pf_ctx* ctx, int form) {
     if (!ctx) return PF_ERR_ARG;
     PF_CHECK(form >= PF_PCG_SCALINGCG && form <= PF_PCG_SINGLE_REDUCTION_RECOMPUTED, PF_ERR_ARG, "pf_set_pcg_form: unknown form");
     ctx->pcg_form = form;
+    return PF_OK;
+}
+
+int pf_set_resident(pf_ctx* ctx, int mode, int after) {
+    if (!ctx) return PF_ERR_ARG;
+    PF_CHECK(mode >= PF_RESIDENT_AUTO && mode <= PF_RESIDENT_STALL && after >= 0, PF_ERR_ARG,
+             "pf_set_resident: unknown mode");
+    ctx->res_mode = mode;
+    ctx->res_after = after;
+    ctx->res_stalled = false;
+    return PF_OK;
+}
+
+int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled) {
+    if (!ctx) return PF_ERR_ARG;
+    if (done) *done = ctx->res_done;
+    if (stalled) *stalled = ctx->res_stalls;
     return PF_OK;
 }
 

@@ -134,6 +134,8 @@ struct pf_ctx {
     unsigned res_tag = 1;
     int res_wgs = 0;
     bool res_stalled = false;
+    int res_mode = PF_RESIDENT_AUTO, res_after = 0;  // pf_set_resident
+    int64_t res_done = 0, res_stalls = 0;            // pf_resident_runs
 
     // MMA state
     struct MmaState* mma = nullptr;

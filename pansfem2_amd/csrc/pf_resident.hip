@@ -650,4 +650,9 @@ __global__ void k_res_start(PcgDev* __restrict__ S, ResDev* __restrict__ R) {
     *R = ResDev{};
 }
 
+// What a workgroup that has waited too long does, before a launch of its own:
+// that launch's workgroups leave at once or as after any solve, and the host
+// goes on with the launched kernels.
+__global__ void k_res_stall(ResDev* __restrict__ R) { R->stall = 1; }
+
 }  // namespace pf

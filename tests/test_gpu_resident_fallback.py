@@ -1,0 +1,110 @@
+"""What follows when a resident kernel gives up: the launched kernels start the
+call over and give the bits that they give with the resident ones switched off,
+whether the resident kernel had written nothing (its first launch) or a partial
+x (a later one).  PF_RESIDENT_STALL marks a launch as stalled from the host, so
+that every kernel ends normally."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pa():
+    import pansfem2_amd
+    return pansfem2_amd
+
+
+def problem(pa, dims):
+    ctx = (pa.cantilever2d if len(dims) == 2 else pa.cantilever3d)(*dims)
+    rng = np.random.default_rng(sum(dims))
+    ctx.set_density(rng.uniform(0.2, 1.0, ctx.ne))
+    return ctx, ctx.load() + rng.uniform(-1e-3, 1e-3, ctx.N)
+
+
+# (after, eps, itrmax): the first launch, or the second one of a solve that takes 2200 iterations
+FIRST, SECOND = (0, 1e-10, 100000), (1, 0.0, 2200)
+
+
+@pytest.mark.parametrize("dims,form,op,when", [
+    ((120, 40), 0, "EBE64", FIRST), ((120, 40), 2, "EBE64", FIRST), ((301, 149), 0, "EBE64", FIRST),
+    ((9, 5, 3), 0, "EBE64", FIRST), ((33, 16, 16), 0, "EBE64", FIRST),
+    ((120, 40), 0, "EBE64", SECOND), ((301, 149), 2, "EBE64", SECOND), ((60, 6, 5), 0, "EBE64", SECOND),
+    ((120, 40), 0, "EBE32", FIRST), ((33, 16, 16), 0, "EBE32", FIRST)])
+def test_stalled_solve(pa, dims, form, op, when):
+    after, eps, itrmax = when
+    print(f"stalled solve {dims} form {form} {op} after {after}", flush=True)
+    ctx, b = problem(pa, dims)
+    ctx.set_pcg_form(form)
+    op = getattr(pa, "PF_OP_" + op)
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
+    ref, sref = ctx.pcg(b, op=op, eps=eps, itrmax=itrmax)
+    assert ctx.resident_runs() == (0, 0)
+    ctx.set_resident(pa.PF_RESIDENT_STALL, after)
+    x, st = ctx.pcg(b, op=op, eps=eps, itrmax=itrmax)
+    assert ctx.resident_runs() == (0, 1)
+    assert st["status"] == sref["status"]
+    if op == pa.PF_OP_EBE64:  # a mixed hex8 solve aims further when it starts resident
+        assert st["iterations"] == sref["iterations"] and np.array_equal(x, ref)
+    else:
+        assert st["true_residual"] <= 1.0000001 * eps
+    # back to the default: resident again
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx.pcg(b, op=op, eps=eps, itrmax=itrmax)
+    assert ctx.resident_runs()[0] >= 1 and ctx.resident_runs()[1] == 1
+    ctx.close()
+
+
+@pytest.mark.parametrize("dims", [(1, 1), (40, 13), (363, 361), (5, 3, 4)])
+def test_stalled_oc_update(pa, dims):
+    ctx, _ = problem(pa, dims)
+    rng = np.random.default_rng(3)
+    x, df, dg = rng.uniform(0.2, 0.8, ctx.ne), -rng.uniform(0.05, 2.0, ctx.ne), rng.uniform(0.5, 1.5, ctx.ne) / ctx.ne
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
+    ref = ctx.oc_update(x, df, dg)
+    capped = ctx.oc_update(x, df, dg, max_steps=7)
+    ctx.set_resident(pa.PF_RESIDENT_STALL)
+    got = ctx.oc_update(x, df, dg)
+    assert ctx.resident_runs() == (0, 1)
+    assert np.array_equal(got[0], ref[0]) and got[1:] == ref[1:]
+    # and the resident bisection itself: the same decisions
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    for want, kw in ((ref, {}), (capped, dict(max_steps=7))):
+        got = ctx.oc_update(x, df, dg, **kw)
+        assert got[1:] == want[1:] and np.max(np.abs(got[0] - want[0])) < 1e-15
+    assert ctx.resident_runs() == (2, 1)
+    ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["mma", "conlin"])
+@pytest.mark.parametrize("n", [(3, 1), (120, 40)])
+def test_stalled_mma_update(pa, n, kind):
+    rng = np.random.default_rng(5)
+    ne = n[0] * n[1]
+    calls = [(-rng.uniform(0.1, 2.0, ne), np.full(ne, 2.0 / ne)) for _ in range(3)]
+    out = {}
+    for mode in (pa.PF_RESIDENT_OFF, pa.PF_RESIDENT_STALL):
+        ctx = pa.cantilever2d(*n)
+        (ctx.mma_init if kind == "mma" else ctx.conlin_init)()
+        update = ctx.mma_update if kind == "mma" else ctx.conlin_update
+        x, steps = np.full(ne, 0.5), []
+        for k, (df, dg) in enumerate(calls):
+            ctx.set_resident(mode)  # a stall sends what follows to the launched kernels
+            x, s = update(x, 1.0, df, float(2.0 * x.mean() - 1.0), dg)
+            steps.append(s)
+        st = ctx.mma_get_state()
+        assert ctx.resident_runs() == (0, 0 if mode == pa.PF_RESIDENT_OFF else len(calls))
+        out[mode] = (x, steps, st["k"], st["xkm1"], st["xkm2"], st["L"], st["U"])
+        ctx.close()
+    a, b = out.values()
+    assert a[1] == b[1] and a[2] == b[2] == len(calls)
+    for i in (0, 3, 4) + ((5, 6) if kind == "mma" else ()):
+        assert np.array_equal(a[i], b[i])
+
+
+def test_mode_argument_checked(pa):
+    ctx = pa.cantilever2d(8, 4)
+    for mode, after in ((3, 0), (-1, 0), (2, -1)):
+        with pytest.raises(pa.PfError):
+            ctx.set_resident(mode, after)
+    ctx.close()

@@ -1,7 +1,9 @@
 """GPU parity of the single-reduction Jacobi-PCG forms (Chronopoulos and
-Gear's recurrences, one launch per iteration; s = K p carried as a vector or
-recomputed on a two-node tile halo) against the reference's ScalingCG results
-and against the device's ScalingCG-order form.
+Gear's recurrences; s = K p carried as a vector or recomputed on a two-node
+tile halo) against the reference's ScalingCG results and against the device's
+ScalingCG-order form.  The carried form and ScalingCG's order run in the
+resident kernel by default and in launched ones (one launch per iteration)
+with it switched off: both are tested, the recomputed form is always launched.
 
 Bars as for ScalingCG itself: displacement within 1e-8 of the reference's at
 eps = 1e-10; the 50-iteration SIMP loop within 1e-9 (compliance) and 1e-6
@@ -33,17 +35,19 @@ def close_counts(a, b):
     return abs(a - b) <= max(3, 0.005 * b)
 
 
-FORMS = [2, 3]  # PF_PCG_SINGLE_REDUCTION_CARRIED, PF_PCG_SINGLE_REDUCTION_RECOMPUTED
+# PF_PCG_SINGLE_REDUCTION_CARRIED, PF_PCG_SINGLE_REDUCTION_RECOMPUTED, and PF_RESIDENT_AUTO or PF_RESIDENT_OFF
+FORMS = [(2, 0), (2, 1), (3, 1)]
 
 
-@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("form,mode", FORMS)
 @pytest.mark.parametrize("case", ["simp_4x2_oc", "simp_8x4_oc", "simp_120x40_oc"])
-def test_solve_against_reference(pa, case, form):
+def test_solve_against_reference(pa, case, form, mode):
     from oracle import pyoracle as po
     g = gi.load(case)
     m = gi.meta(case)
-    print(f"single-reduction solve {case} form {form}", flush=True)
+    print(f"single-reduction solve {case} form {form} mode {mode}", flush=True)
     ctx = pa.cantilever2d(m["nx"], m["ny"])
+    ctx.set_resident(mode)
     ctx.set_density(g["rho0"])
     ctx.set_pcg_form(form)
     u, st = ctx.pcg(g["F"], op=pa.PF_OP_EBE64, eps=1e-10)
@@ -55,14 +59,15 @@ def test_solve_against_reference(pa, case, form):
     ctx.close()
 
 
-@pytest.mark.parametrize("form", FORMS)
-def test_simp_loop_c1_against_reference(pa, form):
+@pytest.mark.parametrize("form,mode", FORMS)
+def test_simp_loop_c1_against_reference(pa, form, mode):
     """50 OC iterations at 120x40 with the single-reduction solver."""
     from oracle import pyoracle as po
     case = "simp_120x40_oc"
     g = gi.load(case)
-    print(f"single-reduction SIMP loop 120x40 form {form}", flush=True)
+    print(f"single-reduction SIMP loop 120x40 form {form} mode {mode}", flush=True)
     ctx = pa.cantilever2d(120, 40)
+    ctx.set_resident(mode)
     ctx.set_pcg_form(form)
     r = ctx.simp_run(50)
     ref = po.simp2d(120, 40, 50)
@@ -74,12 +79,13 @@ def test_simp_loop_c1_against_reference(pa, form):
     ctx.close()
 
 
-@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("form,mode", FORMS)
 @pytest.mark.parametrize("nx,ny", [(127, 63), (135, 70), (1024, 512)])
-def test_agrees_with_scalingcg_order(pa, nx, ny, form):
+def test_agrees_with_scalingcg_order(pa, nx, ny, form, mode):
     """Beyond the oracle's sizes: both forms on an i.i.d. density field."""
-    print(f"single-reduction vs ScalingCG order {nx}x{ny} form {form}", flush=True)
+    print(f"single-reduction vs ScalingCG order {nx}x{ny} form {form} mode {mode}", flush=True)
     ctx = pa.cantilever2d(nx, ny)
+    ctx.set_resident(mode)
     rng = np.random.default_rng(20261206)
     ctx.set_density(rng.uniform(1e-3, 1.0, nx * ny))
     b = ctx.load()
@@ -98,9 +104,10 @@ def test_agrees_with_scalingcg_order(pa, nx, ny, form):
     ctx.close()
 
 
-@pytest.mark.parametrize("form", FORMS)
-def test_zero_load_and_itrmax_exit(pa, form):
+@pytest.mark.parametrize("form,mode", FORMS)
+def test_zero_load_and_itrmax_exit(pa, form, mode):
     ctx = pa.cantilever2d(64, 32)
+    ctx.set_resident(mode)
     rng = np.random.default_rng(5)
     ctx.set_density(rng.uniform(0.1, 1.0, 64 * 32))
     b = ctx.load()
@@ -125,8 +132,10 @@ def test_zero_load_and_itrmax_exit(pa, form):
 
 def test_automatic_form_takes_the_carried_kernel_below_150_mb(pa):
     """PF_PCG_SINGLE_REDUCTION at 1024x512 (an 80 MB working set) runs the
-    carried kernel: the same bits as PF_PCG_SINGLE_REDUCTION_CARRIED."""
+    carried kernel where it is launched: the same bits as
+    PF_PCG_SINGLE_REDUCTION_CARRIED, and not those of the recomputed form."""
     ctx = pa.cantilever2d(1024, 512)
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
     rng = np.random.default_rng(11)
     ctx.set_density(rng.uniform(1e-3, 1.0, ctx.ne))
     b = ctx.load()
@@ -135,6 +144,9 @@ def test_automatic_form_takes_the_carried_kernel_below_150_mb(pa):
     ctx.set_pcg_form(pa.PF_PCG_SINGLE_REDUCTION_CARRIED)
     x2, s2 = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-6)
     assert s1["iterations"] == s2["iterations"] and np.array_equal(x1, x2)
+    ctx.set_pcg_form(pa.PF_PCG_SINGLE_REDUCTION_RECOMPUTED)
+    assert not np.array_equal(x1, ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-6)[0])
+    assert ctx.resident_runs() == (0, 0)
     ctx.close()
 
 
