@@ -214,7 +214,8 @@ int pf_set_pcg_form(pf_ctx* ctx, int form);
  * fits the chip, and in kernels launched per iteration (per Newton or bisection
  * step) otherwise: on larger grids, where a cooperative launch is refused, and
  * after a resident kernel's workgroups have waited two seconds for one
- * another (a stall; the call then starts over).  Until changed:
+ * another (a stall: the call starts over, and so does the next call, after a
+ * second stall in a row the next two, up to 1024).  Until changed:
  *   PF_RESIDENT_AUTO: so (the default);
  *   PF_RESIDENT_OFF: always launched;
  *   PF_RESIDENT_STALL: as AUTO, but a resident solve's launches (2048

@@ -259,6 +259,7 @@ void free_grid(pf_ctx* ctx) {
     dfree(ctx->res_halo);
     dfree(ctx->res_loc);
     ctx->res_halo_n = ctx->res_loc_n = 0;
+    ctx->res_pause = ctx->res_backoff = 0;
     dfree(ctx->d_e0); dfree(ctx->d_e1); dfree(ctx->d_e2); dfree(ctx->d_e3); dfree(ctx->d_e4); dfree(ctx->d_e5);
     dfree(ctx->d_e6);
     dfree(ctx->d_cg); dfree(ctx->d_load);
@@ -478,18 +479,30 @@ const void* res_kernel(const ResShape& sh) {
 
 // whether this context's solves and updates may run resident
 bool res_on(const pf_ctx* ctx) {
-    return ctx->res_wgs >= 1 && ctx->res_mode != PF_RESIDENT_OFF && !ctx->res_stalled;
+    return ctx->res_wgs >= 1 && ctx->res_mode != PF_RESIDENT_OFF && ctx->res_pause == 0;
+}
+// At the start of a solve, update or bisection that may: one call less to wait
+// after a stall.
+void res_enter(pf_ctx* ctx) {
+    if (ctx->res_pause > 0) ctx->res_pause--;
 }
 // Before launch number `launch` of a resident solve: PF_RESIDENT_STALL's flag.
 void res_force(pf_ctx* ctx, int launch) {
     if (ctx->res_mode == PF_RESIDENT_STALL && launch >= ctx->res_after) k_res_stall<<<1, 1, 0, ctx->stream>>>(ctx->d_res);
 }
-// After a resident launch (h_res copied back): whether a workgroup gave up.
+// After a resident launch (h_res copied back): whether a workgroup gave up.  The
+// next call is then launched, after a second stall in a row the next two, and
+// so on up to 1024: what keeps the GPU busy may end, and a stall costs 2 s.
 bool res_gave_up(pf_ctx* ctx) {
     if (!ctx->h_res->stall) return false;
-    ctx->res_stalled = true;
+    ctx->res_backoff = std::min(1024, std::max(1, 2 * ctx->res_backoff));
+    ctx->res_pause = ctx->res_backoff + 1;  // res_enter of the call that tries again takes the last one
     ctx->res_stalls++;
     return true;
+}
+void res_ended(pf_ctx* ctx) {
+    ctx->res_backoff = 0;
+    ctx->res_done++;
 }
 
 constexpr int kResChunk = 2048;  // iterations per launch: other streams get the GPU in between
@@ -546,7 +559,7 @@ int res_run(pf_ctx* ctx, const void* kern, int wgs, int nt, size_t lds, ARGS& A,
         if (H->done || m >= end) break;
     }
     *ran = true;
-    ctx->res_done++;
+    res_ended(ctx);
     out.iterations = H->iterations;
     out.status = H->status;
     out.rnorm = H->rnorm;
@@ -2643,6 +2656,7 @@ int solve_nodal(pf_ctx* ctx, int op, const double* b, double* x, double eps, int
             return PF_OK;
         }
     }
+    if (op == PF_OP_EBE64 || op == PF_OP_EBE32) res_enter(ctx);
     if (op == PF_OP_EBE64) {
         PF_TRY(diag_nodal(ctx, false));
         PcgRun run;
@@ -2755,7 +2769,7 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_TRY(sync(ctx));
     if (res_gave_up(ctx)) return PF_OK;
-    ctx->res_done++;
+    res_ended(ctx);
     *ran = true;
     return PF_OK;
 }
@@ -2767,6 +2781,7 @@ int oc_device(pf_ctx* ctx, const pf_oc_params* prm, const double* x, const doubl
     OcDev* S = (OcDev*)ctx->d_oc;
     const int max_steps = prm->max_steps > 0 ? prm->max_steps : 200;
     bool resident;
+    res_enter(ctx);
     PF_TRY(oc_resident(ctx, prm, max_steps, x, dfdx, dgdx, xplus, &resident));
     if (!resident) {
         OcDev init{};
@@ -2974,7 +2989,7 @@ int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, c
     PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_TRY(sync(ctx));
     if (res_gave_up(ctx)) return PF_OK;
-    ctx->res_done++;
+    res_ended(ctx);
     *steps = (int)ctx->h_res->v[0];
     *status = (int)ctx->h_res->v[1];
     *ran = true;
@@ -3004,6 +3019,7 @@ int mma_update_device(pf_ctx* ctx, double* xk, double f, const double* dfdx, dou
     {
         int steps = 0, status = 0;
         bool ran;
+        res_enter(ctx);
         PF_TRY(mma_update_resident(ctx, xk, dfdx, g, dgdx, &steps, &status, &ran));
         if (ran) {
             if (steps_out) *steps_out = steps;
@@ -3680,7 +3696,6 @@ int pf_set_resident(pf_ctx* ctx, int mode, int after) {
              "pf_set_resident: unknown mode");
     ctx->res_mode = mode;
     ctx->res_after = after;
-    ctx->res_stalled = false;
     return PF_OK;
 }
 

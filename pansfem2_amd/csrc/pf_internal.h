@@ -125,15 +125,14 @@ struct pf_ctx {
 
     // resident solves (pf_resident.hip): exchange buffers and scalars between
     // launches (slots, d_res and h_res are parts of red.partials and h_red),
-    // the next unused exchange tag, the workgroups that run at once (0: none),
-    // and whether a solve stalled (this context then launches)
+    // the next unused exchange tag and the workgroups that run at once (0: none)
     unsigned long long *res_slots = nullptr, *res_halo = nullptr;
     double* res_loc = nullptr;              // hex8: the workgroups' own x
     long res_halo_n = 0, res_loc_n = 0;     // their sizes
     pf::ResDev *d_res = nullptr, *h_res = nullptr;
     unsigned res_tag = 1;
     int res_wgs = 0;
-    bool res_stalled = false;
+    int res_pause = 0, res_backoff = 0;  // calls still to be launched after a stall (res_gave_up)
     int res_mode = PF_RESIDENT_AUTO, res_after = 0;  // pf_set_resident
     int64_t res_done = 0, res_stalls = 0;            // pf_resident_runs
 

@@ -15,8 +15,8 @@ def pa():
     return pansfem2_amd
 
 
-def problem(pa, dims):
-    ctx = (pa.cantilever2d if len(dims) == 2 else pa.cantilever3d)(*dims)
+def problem(pa, dims, ctx=None):
+    ctx = (pa.cantilever2d if len(dims) == 2 else pa.cantilever3d)(*dims, ctx=ctx)
     rng = np.random.default_rng(sum(dims))
     ctx.set_density(rng.uniform(0.2, 1.0, ctx.ne))
     return ctx, ctx.load() + rng.uniform(-1e-3, 1e-3, ctx.N)
@@ -48,10 +48,42 @@ def test_stalled_solve(pa, dims, form, op, when):
         assert st["iterations"] == sref["iterations"] and np.array_equal(x, ref)
     else:
         assert st["true_residual"] <= 1.0000001 * eps
-    # back to the default: resident again
+    ctx.close()
+
+
+def test_calls_after_stalls_are_launched_and_then_tried_again(pa):
+    """One call after the first stall, two after the second in a row, four after
+    the third; a solve that ends resident, or a new grid, ends the count."""
+    ctx, b = problem(pa, (40, 13))
+    solve = lambda: ctx.pcg(b, eps=1e-8)[1]["status"] == 1  # noqa: E731
+    runs = []
+    ctx.set_resident(pa.PF_RESIDENT_STALL)
+    for _ in range(10):
+        assert solve()
+        runs.append(ctx.resident_runs())
+    assert runs == [(0, k) for k in (1, 1, 2, 2, 2, 3, 3, 3, 3, 3)]
     ctx.set_resident(pa.PF_RESIDENT_AUTO)
-    ctx.pcg(b, op=op, eps=eps, itrmax=itrmax)
-    assert ctx.resident_runs()[0] >= 1 and ctx.resident_runs()[1] == 1
+    assert solve() and solve() and ctx.resident_runs() == (2, 3)
+    ctx.set_resident(pa.PF_RESIDENT_STALL)
+    assert solve() and solve() and ctx.resident_runs() == (2, 4)
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    assert solve() and ctx.resident_runs() == (3, 4)
+    # updates and bisections count as calls, solves that cannot run resident do not
+    ctx.set_resident(pa.PF_RESIDENT_STALL)
+    assert solve() and ctx.resident_runs() == (3, 5)
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx.assemble_csr()
+    ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-8)
+    x, g = np.full(ctx.ne, 0.5), np.full(ctx.ne, 1.0 / ctx.ne)
+    ctx.oc_update(x, -g, g)
+    assert ctx.resident_runs() == (3, 5)
+    ctx.oc_update(x, -g, g)
+    assert ctx.resident_runs() == (4, 5)
+    ctx.set_resident(pa.PF_RESIDENT_STALL)
+    assert solve() and ctx.resident_runs() == (4, 6)
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx, b = problem(pa, (33, 13), ctx)
+    assert solve() and ctx.resident_runs() == (5, 6)
     ctx.close()
 
 
@@ -67,8 +99,9 @@ def test_stalled_oc_update(pa, dims):
     got = ctx.oc_update(x, df, dg)
     assert ctx.resident_runs() == (0, 1)
     assert np.array_equal(got[0], ref[0]) and got[1:] == ref[1:]
-    # and the resident bisection itself: the same decisions
+    # and the resident bisection itself, two calls later: the same decisions
     ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx.oc_update(x, df, dg)
     for want, kw in ((ref, {}), (capped, dict(max_steps=7))):
         got = ctx.oc_update(x, df, dg, **kw)
         assert got[1:] == want[1:] and np.max(np.abs(got[0] - want[0])) < 1e-15
@@ -89,11 +122,11 @@ def test_stalled_mma_update(pa, n, kind):
         update = ctx.mma_update if kind == "mma" else ctx.conlin_update
         x, steps = np.full(ne, 0.5), []
         for k, (df, dg) in enumerate(calls):
-            ctx.set_resident(mode)  # a stall sends what follows to the launched kernels
+            ctx.set_resident(mode)
             x, s = update(x, 1.0, df, float(2.0 * x.mean() - 1.0), dg)
             steps.append(s)
         st = ctx.mma_get_state()
-        assert ctx.resident_runs() == (0, 0 if mode == pa.PF_RESIDENT_OFF else len(calls))
+        assert ctx.resident_runs() == (0, 0 if mode == pa.PF_RESIDENT_OFF else 2)  # the second call is launched
         out[mode] = (x, steps, st["k"], st["xkm1"], st["xkm2"], st["L"], st["U"])
         ctx.close()
     a, b = out.values()
