@@ -212,18 +212,21 @@ int pf_set_pcg_form(pf_ctx* ctx, int form);
 /* Jacobi-PCG solves with the matrix-free operators, MMA and CONLIN updates and
  * OC bisections without projection run in one resident kernel where the grid
  * fits the chip, and in kernels launched per iteration (per Newton or bisection
- * step) otherwise: on larger grids, where a cooperative launch is refused, and
- * after a resident kernel's workgroups have waited two seconds for one
- * another (a stall: the call starts over, and so does the next call, after a
- * second stall in a row the next two, up to 1024).  Until changed:
+ * step) otherwise: on larger grids, where a cooperative launch is refused or
+ * the resident kernel's buffers cannot be had, and after a stall (a resident
+ * kernel's workgroups have waited two seconds for one another): the call then
+ * starts over launched, and so does the next one run, after a second stall in
+ * a row the next two, and so on up to 1024.  Until changed:
  *   PF_RESIDENT_AUTO: so (the default);
  *   PF_RESIDENT_OFF: always launched;
  *   PF_RESIDENT_STALL: as AUTO, but a resident solve's launches (2048
  *     iterations each; an update or bisection is one launch) after the first
- *     `after` end as stalled, as beside a program that keeps the GPU busy: for
- *     tests of what follows.
- * `after` is not used by the other modes.  Has no counterpart in the reference. */
-enum { PF_RESIDENT_AUTO = 0, PF_RESIDENT_OFF = 1, PF_RESIDENT_STALL = 2 };
+ *     `after` end as stalled, as beside a program that keeps the GPU busy;
+ *   PF_RESIDENT_NOMEM: as AUTO, but of the buffers that resident kernels still
+ *     have to allocate, those after the first `after` are not to be had.
+ * The last two are for tests of what follows; the others do not use `after`.
+ * Has no counterpart in the reference. */
+enum { PF_RESIDENT_AUTO = 0, PF_RESIDENT_OFF = 1, PF_RESIDENT_STALL = 2, PF_RESIDENT_NOMEM = 3 };
 int pf_set_resident(pf_ctx* ctx, int mode, int after);
 /* How many solves (inner solves of a mixed one each), updates and bisections
  * of this context have run resident to their end, and how many have stalled. */

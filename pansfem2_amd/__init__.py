@@ -21,7 +21,7 @@ PF_PCG_SINGLE_REDUCTION_CARRIED, PF_PCG_SINGLE_REDUCTION_RECOMPUTED = 2, 3
 PF_MG_PROLONG_BILINEAR, PF_MG_PROLONG_STIFFNESS = 0, 1
 PF_MG_RESIDUAL_AUTO, PF_MG_RESIDUAL_NODE, PF_MG_RESIDUAL_ELEMENT = 0, 1, 2
 PF_H8_OP_VALU, PF_H8_OP_MFMA = 0, 1
-PF_RESIDENT_AUTO, PF_RESIDENT_OFF, PF_RESIDENT_STALL = 0, 1, 2
+PF_RESIDENT_AUTO, PF_RESIDENT_OFF, PF_RESIDENT_STALL, PF_RESIDENT_NOMEM = 0, 1, 2, 3
 
 _i32p = np.ctypeslib.ndpointer(np.int32, flags="C_CONTIGUOUS")
 _f64p = np.ctypeslib.ndpointer(np.float64, flags="C_CONTIGUOUS")
@@ -357,9 +357,10 @@ class Context:
     def set_resident(self, mode, after=0):
         """PF_RESIDENT_AUTO (the default: one resident kernel per solve, MMA /
         CONLIN update and OC bisection where the grid fits the chip),
-        PF_RESIDENT_OFF (always the launched kernels) or PF_RESIDENT_STALL
-        (resident launches after the first `after` of a solve end as stalled:
-        for tests of the fallback)."""
+        PF_RESIDENT_OFF (always the launched kernels); for tests of the
+        fallback PF_RESIDENT_STALL (resident launches after the first `after`
+        of a solve end as stalled) and PF_RESIDENT_NOMEM (the buffers they
+        allocate after the first `after` cannot be had)."""
         self._ck(lib().pf_set_resident(self._h, mode, after))
 
     def resident_runs(self):

@@ -271,6 +271,7 @@ void free_grid(pf_ctx* ctx) {
     ctx->have_filter = false;
     ctx->have_lists = false;
     dfree(ctx->d_fcol);
+    ctx->fcol_n = 0;
     ctx->have_fcol = false;
     release_net(ctx);
 }
@@ -507,15 +508,30 @@ void res_ended(pf_ctx* ctx) {
 
 constexpr int kResChunk = 2048;  // iterations per launch: other streams get the GPU in between
 
-// Exchange buffer of `words` words for a solve that starts now, and the
-// solve's scalars.
-int res_begin(pf_ctx* ctx, long words) {
-    const bool fresh = ctx->res_halo_n < words;
-    if (fresh) {
-        ctx->res_halo_n = 0;
-        PF_TRY(dalloc(ctx, &ctx->res_halo, words));
-        ctx->res_halo_n = words;
+// A buffer that only a resident kernel needs, of at least n values (*have: its
+// size); false when it cannot be had, which is no error: the launched kernels
+// do without.
+template <class T>
+bool res_alloc(pf_ctx* ctx, T** p, long n, long* have) {
+    if (*have >= n) return true;
+    dfree(*p);
+    *have = 0;
+    if (ctx->res_mode == PF_RESIDENT_NOMEM && ctx->res_after-- <= 0) return false;
+    if (hipMalloc((void**)p, sizeof(T) * (size_t)n) != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+        return false;
     }
+    *have = n;
+    return true;
+}
+
+// Exchange buffer of `words` words for a solve that starts now, and the
+// solve's scalars; *ok false: it cannot be had.
+int res_begin(pf_ctx* ctx, long words, bool* ok) {
+    const bool fresh = ctx->res_halo_n < words;
+    *ok = res_alloc(ctx, &ctx->res_halo, words, &ctx->res_halo_n);
+    if (!*ok) return PF_OK;
     if (fresh || ctx->res_tag > 0xf0000000u) {
         // no word may carry a tag that is still to come
         k_fill<u64><<<gsize(words), kBlock, 0, ctx->stream>>>(ctx->res_halo_n, ctx->res_halo, 0ull);
@@ -586,7 +602,9 @@ int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s,
     if (!sh.gi) return PF_OK;
     const void* kern = sr ? res_kernel<T, true>(sh) : res_kernel<T, false>(sh);
     if (!res_lds_ok(kern, sh.lds)) return PF_OK;
-    PF_TRY(res_begin(ctx, 2 * ctx->nn * 4));
+    bool ok;
+    PF_TRY(res_begin(ctx, 2 * ctx->nn * 4, &ok));
+    if (!ok) return PF_OK;
     const bool f32 = std::is_same<T, float>::value;
     ResArgs<T> A{};
     A.nx = ctx->nx; A.ny = ctx->ny; A.gi = sh.gi; A.gj = sh.gj;
@@ -663,13 +681,10 @@ int pcg_resident3(pf_ctx* ctx, const T* b, T* x, const T* D, T* r, T* p, double 
                                      : (const void*)k_pcg_h8_resident<T, kRes3Slots>;
     if (!res_lds_ok(kern, sh.lds)) return PF_OK;
     const int wgs = sh.gi * sh.gj * sh.gk;
-    PF_TRY(res_begin(ctx, 2L * wgs * sh.box));
     const long local = (long)wgs * kRes3Threads * sh.slots;  // x of every workgroup's values
-    if (ctx->res_loc_n < local) {
-        ctx->res_loc_n = 0;
-        PF_TRY(dalloc(ctx, &ctx->res_loc, local));
-        ctx->res_loc_n = local;
-    }
+    bool ok;
+    PF_TRY(res_begin(ctx, 2L * wgs * sh.box, &ok));
+    if (!ok || !res_alloc(ctx, &ctx->res_loc, local, &ctx->res_loc_n)) return PF_OK;
     const bool f32 = std::is_same<T, float>::value;
     Res3Args<T> A{};
     A.nx = ctx->nx; A.ny = ctx->ny; A.nz = ctx->nz;
@@ -2720,8 +2735,8 @@ int solve_nodal(pf_ctx* ctx, int op, const double* b, double* x, double eps, int
 // ------------------------------------------------------------------ OC ----
 // The bisection in one resident launch (k_oc_resident), its result in h_oc;
 // *ran is false, and nothing has been done, with the projection in the closure,
-// more elements than the chip's registers hold or a launch that cannot be made
-// or stalled.
+// more elements than the chip's registers hold, no memory for the column sums or
+// a launch that cannot be made or stalled.
 int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const double* x, const double* dfdx,
                 const double* dgdx, double* xplus, bool* ran) {
     *ran = false;
@@ -2729,7 +2744,7 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     const long ne = ctx->ne, most = (long)ctx->res_wgs * NT;
     if (!res_on(ctx) || ne > 16 * most || prm->beta > 0.0 || max_steps > 1000000) return PF_OK;
     if (!ctx->have_fcol) {
-        if (!ctx->d_fcol) PF_TRY(dalloc(ctx, &ctx->d_fcol, ne));
+        if (!res_alloc(ctx, &ctx->d_fcol, ne, &ctx->fcol_n)) return PF_OK;
         k_filter_colsum<<<gsize(ne), kBlock, 0, ctx->stream>>>(g3(ctx), ctx->dim, ctx->win, ctx->R, ctx->d_cg, nullptr,
                                                                xplus);
         k_filter_colsum<<<gsize(ne), kBlock, 0, ctx->stream>>>(g3(ctx), ctx->dim, ctx->win, ctx->R, ctx->d_cg, xplus,
@@ -2745,7 +2760,8 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
                        : S == 4 ? (const void*)k_oc_resident<4>
                        : S == 8 ? (const void*)k_oc_resident<8>
                                 : (const void*)k_oc_resident<16>;
-    PF_TRY(res_begin(ctx, 0));
+    bool ok;
+    PF_TRY(res_begin(ctx, 0, &ok));  // no buffer of its own
     OcRes A{};
     A.n = ne;
     A.max_steps = max_steps;
@@ -2963,7 +2979,8 @@ int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, c
                                  : (S == 1 ? (const void*)k_mma_resident<1, false>
                                     : S == 2 ? (const void*)k_mma_resident<2, false>
                                              : (const void*)k_mma_resident<4, false>);
-    PF_TRY(res_begin(ctx, 0));
+    bool ok;
+    PF_TRY(res_begin(ctx, 0, &ok));  // no buffer of its own
     MmaRes A{};
     A.n = M->n;
     A.early = M->k < 2;
@@ -3692,7 +3709,7 @@ int pf_set_pcg_form(pf_ctx* ctx, int form) {
 
 int pf_set_resident(pf_ctx* ctx, int mode, int after) {
     if (!ctx) return PF_ERR_ARG;
-    PF_CHECK(mode >= PF_RESIDENT_AUTO && mode <= PF_RESIDENT_STALL && after >= 0, PF_ERR_ARG,
+    PF_CHECK(mode >= PF_RESIDENT_AUTO && mode <= PF_RESIDENT_NOMEM && after >= 0, PF_ERR_ARG,
              "pf_set_resident: unknown mode");
     ctx->res_mode = mode;
     ctx->res_after = after;

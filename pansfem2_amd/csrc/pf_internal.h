@@ -112,6 +112,7 @@ struct pf_ctx {
     bool have_lists = false;
     double* d_fcol = nullptr;  // column sums of the grid rule's normalised weights, formed when an OC update needs them
     bool have_fcol = false;
+    long fcol_n = 0;           // its size
     int32_t *d_fptr = nullptr, *d_fidx = nullptr;
     double* d_fw = nullptr;
 

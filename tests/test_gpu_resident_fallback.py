@@ -135,9 +135,50 @@ def test_stalled_mma_update(pa, n, kind):
         assert np.array_equal(a[i], b[i])
 
 
+@pytest.mark.parametrize("after", [0, 1])
+@pytest.mark.parametrize("dims,op", [((120, 40), "EBE64"), ((120, 40), "EBE32"), ((33, 16, 16), "EBE64"),
+                                     ((33, 16, 16), "EBE32")])
+def test_solve_without_memory_for_the_exchange(pa, dims, op, after):
+    """Resident solves allocate an exchange buffer, on hex8 another for x: where
+    one of them cannot be had the launched kernels solve, which need neither."""
+    if after and len(dims) == 2:
+        pytest.skip("one buffer")
+    ctx, b = problem(pa, dims)
+    op = getattr(pa, "PF_OP_" + op)
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
+    ref, sref = ctx.pcg(b, op=op, eps=1e-9)
+    for _ in range(2):
+        ctx.set_resident(pa.PF_RESIDENT_NOMEM, after)
+        x, st = ctx.pcg(b, op=op, eps=1e-9)
+        assert st["status"] == sref["status"] == 1 and st["true_residual"] < 1e-8
+        if op == pa.PF_OP_EBE64:
+            assert np.array_equal(x, ref)
+        assert ctx.resident_runs() == (0, 0)
+        after = 0  # the exchange buffer is there by now, if it could be had
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx.pcg(b, op=op, eps=1e-9)
+    assert ctx.resident_runs()[0] >= 1
+    ctx.close()
+
+
+def test_oc_update_without_memory_for_the_column_sums(pa):
+    ctx, _ = problem(pa, (40, 13))
+    rng = np.random.default_rng(3)
+    x, df, dg = rng.uniform(0.2, 0.8, ctx.ne), -rng.uniform(0.05, 2.0, ctx.ne), np.full(ctx.ne, 1.0 / ctx.ne)
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
+    ref = ctx.oc_update(x, df, dg)
+    ctx.set_resident(pa.PF_RESIDENT_NOMEM)
+    got = ctx.oc_update(x, df, dg)
+    assert ctx.resident_runs() == (0, 0) and np.array_equal(got[0], ref[0]) and got[1:] == ref[1:]
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx.oc_update(x, df, dg)
+    assert ctx.resident_runs() == (1, 0)
+    ctx.close()
+
+
 def test_mode_argument_checked(pa):
     ctx = pa.cantilever2d(8, 4)
-    for mode, after in ((3, 0), (-1, 0), (2, -1)):
+    for mode, after in ((4, 0), (-1, 0), (2, -1)):
         with pytest.raises(pa.PfError):
             ctx.set_resident(mode, after)
     ctx.close()
