@@ -241,12 +241,12 @@ int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled);
  *   PF_H8_OP_MFMA: the element matrix as a batched product on the matrix
  *     cores (16 elements of one colour per product, K0 in registers), the
  *     rows summed per node in LDS in colour order (deterministic).
- * Until a call chooses one, Jacobi-PCG solves of grids that fit the chip (up
- * to about 128 x 64 x 64 elements) run in one resident kernel, with the
- * element matrix in its parity basis where it has one (any box element of a
- * material with the box's mirror planes), and the others use PF_H8_OP_VALU.
- * Has no counterpart in the reference. */
-enum { PF_H8_OP_VALU = 0, PF_H8_OP_MFMA = 1 };
+ *   PF_H8_OP_AUTO (the default): Jacobi-PCG solves of grids that fit the chip (up
+ *     to about 128 x 64 x 64 elements) run in one resident kernel, with the
+ *     element matrix in its parity basis where it has one (any box element of a
+ *     material with the box's mirror planes), and the others use PF_H8_OP_VALU.
+ * The other two are always launched.  Has no counterpart in the reference. */
+enum { PF_H8_OP_AUTO = -1, PF_H8_OP_VALU = 0, PF_H8_OP_MFMA = 1 };
 int pf_set_h8_operator(pf_ctx* ctx, int kind);
 /* Same on device-resident free-DOF vectors. */
 int pf_pcg_dev(pf_ctx* ctx, int op, const double* b_free_dev, double* x_free_dev, double eps, int itrmax,

@@ -20,7 +20,7 @@ PF_PCG_SCALINGCG, PF_PCG_SINGLE_REDUCTION = 0, 1
 PF_PCG_SINGLE_REDUCTION_CARRIED, PF_PCG_SINGLE_REDUCTION_RECOMPUTED = 2, 3
 PF_MG_PROLONG_BILINEAR, PF_MG_PROLONG_STIFFNESS = 0, 1
 PF_MG_RESIDUAL_AUTO, PF_MG_RESIDUAL_NODE, PF_MG_RESIDUAL_ELEMENT = 0, 1, 2
-PF_H8_OP_VALU, PF_H8_OP_MFMA = 0, 1
+PF_H8_OP_AUTO, PF_H8_OP_VALU, PF_H8_OP_MFMA = -1, 0, 1
 PF_RESIDENT_AUTO, PF_RESIDENT_OFF, PF_RESIDENT_STALL, PF_RESIDENT_NOMEM = 0, 1, 2, 3
 
 _i32p = np.ctypeslib.ndpointer(np.int32, flags="C_CONTIGUOUS")
@@ -370,9 +370,10 @@ class Context:
         return d.value, s.value
 
     def set_h8_operator(self, kind):
-        """PF_H8_OP_VALU (one node per thread on the vector units) or
-        PF_H8_OP_MFMA (the element matrix as a batched product on the matrix
-        cores) for the hex8 fused PCG kernel of this context."""
+        """PF_H8_OP_AUTO (the default: the resident kernel where the grid
+        fits the chip, else PF_H8_OP_VALU), PF_H8_OP_VALU (one node per thread
+        on the vector units) or PF_H8_OP_MFMA (the element matrix as a batched
+        product on the matrix cores) for the hex8 Jacobi-PCG of this context."""
         self._ck(lib().pf_set_h8_operator(self._h, kind))
 
     def pcg(self, b, op=PF_OP_EBE64, eps=1e-10, itrmax=100000):

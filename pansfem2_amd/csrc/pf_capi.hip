@@ -665,7 +665,7 @@ Res3Shape res3_pick(const pf_ctx* ctx) {
 }
 
 bool res3_applies(const pf_ctx* ctx) {
-    return res_on(ctx) && ctx->d_K0p && ctx->h8_op < 0;
+    return res_on(ctx) && ctx->d_K0p && ctx->h8_op == PF_H8_OP_AUTO;
 }
 
 // The same for hex8 (k_pcg_h8_resident), ScalingCG's order; only for an
@@ -3725,7 +3725,8 @@ int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled) {
 
 int pf_set_h8_operator(pf_ctx* ctx, int kind) {
     if (!ctx) return PF_ERR_ARG;
-    PF_CHECK(kind == PF_H8_OP_VALU || kind == PF_H8_OP_MFMA, PF_ERR_ARG, "pf_set_h8_operator: unknown kind");
+    PF_CHECK(kind == PF_H8_OP_AUTO || kind == PF_H8_OP_VALU || kind == PF_H8_OP_MFMA, PF_ERR_ARG,
+             "pf_set_h8_operator: unknown kind");
     ctx->h8_op = kind;
     return PF_OK;
 }

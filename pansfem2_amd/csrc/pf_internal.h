@@ -147,9 +147,7 @@ struct pf_ctx {
     struct MgState* mg = nullptr;
     int mg_prolong = PF_MG_PROLONG_STIFFNESS;
     int mg_resid = PF_MG_RESIDUAL_AUTO;  // hex8 coarse-level residual form
-    // hex8 matrix-free operator of the fused PCG kernel as pf_set_h8_operator
-    // chose it; -1, the default: the resident solve where it fits, else PF_H8_OP_VALU
-    int h8_op = -1;
+    int h8_op = PF_H8_OP_AUTO;  // hex8 matrix-free operator of the Jacobi-PCG (pf_set_h8_operator)
 
     // device address of the library's static scratch array on this
     // context's device (pf_compliance_sens_dev_noalloc)

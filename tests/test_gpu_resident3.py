@@ -113,3 +113,20 @@ def test_element_matrix_without_parity_blocks(pa):
         assert rel(x, xm) < 1e-12
     ctx.close()
     other.close()
+
+
+def test_default_operator_after_another(pa):
+    """PF_H8_OP_AUTO brings a context back to the resident kernel, with the bits
+    that it gave before."""
+    ctx, b = problem(pa, 9, 5, 3)
+    x, _ = ctx.pcg(b, eps=1e-10)
+    for kind in (pa.PF_H8_OP_VALU, pa.PF_H8_OP_MFMA):
+        ctx.set_h8_operator(kind)
+        ran = ctx.resident_runs()[0]
+        assert rel(ctx.pcg(b, eps=1e-10)[0], x) < 1e-8 and ctx.resident_runs()[0] == ran
+        ctx.set_h8_operator(pa.PF_H8_OP_AUTO)
+        assert np.array_equal(ctx.pcg(b, eps=1e-10)[0], x) and ctx.resident_runs()[0] == ran + 1
+    for kind in (-2, 2):
+        with pytest.raises(pa.PfError):
+            ctx.set_h8_operator(kind)
+    ctx.close()
