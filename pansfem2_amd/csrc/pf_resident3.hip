@@ -156,10 +156,13 @@ __device__ inline float res_row_up(float v) {
 }
 
 // The two words of a double in one 16-byte store (each word is read by itself).
+// A store of more than 8 bytes must be two wait states ahead of the next write
+// of its data registers; the compiler does not see the store in the asm, so the
+// s_nop is in it too.
 __device__ inline void res_put2(u64* p, unsigned tag, double v) {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     const u4 w = {res_half(v, 0), tag, res_half(v, 1), tag};
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(w) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(w) : "memory");
 }
 
 constexpr int kRes3Threads = 512;
