@@ -3420,6 +3420,8 @@ int pf_set_element_matrix(pf_ctx* ctx, const double* K0, int nd) {
         const bool parity = h8_parity_pack(K0, m64.data() + 768);
         for (int i = 0; i < kH8ParityCoefs; i++) m32[768 + i] = (float)m64[768 + i];
         const long nm = (long)m64.size();
+        ctx->d_K0p = nullptr;  // inside d_K0m and d_K0mf, which the next lines free
+        ctx->d_K0pf = nullptr;
         PF_TRY(dalloc(ctx, &ctx->d_K0m, nm));
         PF_TRY(dalloc(ctx, &ctx->d_K0mf, nm));
         PF_HIP(hipMemcpyAsync(ctx->d_K0m, m64.data(), sizeof(double) * nm, hipMemcpyHostToDevice, ctx->stream));
