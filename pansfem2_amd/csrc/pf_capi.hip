@@ -956,7 +956,9 @@ double norm_nodal(pf_ctx* ctx, const double* a, int* rc) {
 // 2.3e-8 off in the mean, 1.9e-9 with the direct operator in one more step.
 // There both are tightened to an eighth, which gives 8e-10 in 23 to 39 ms
 // (launched 102 to 143 ms, untightened 18 to 35 ms); a last step solves no
-// further than it has to.
+// further than it has to, and one that starts with the caller's tolerance met
+// takes no more iterations than the longest before it (where FP32 cannot
+// reach the eighth it would run to kInnerCap to be undone).
 int pcg_ir(pf_ctx* ctx, const double* b, double* x, double eps, int itrmax, double inner_eps, pf_solve_stats& st) {
     constexpr int kInnerCap = 20000;
     const bool parity = !is2d(ctx) && res3_applies(ctx) && res3_pick<float>(ctx).gi > 0;
@@ -967,22 +969,25 @@ int pcg_ir(pf_ctx* ctx, const double* b, double* x, double eps, int itrmax, doub
     PF_TRY(rc);
     PF_HIP(hipMemsetAsync(x, 0, sizeof(double) * ctx->nv, ctx->stream));
     double rn = bn;
-    int outer = 0, total = 0, status = 2, fallbacks = 0;
+    int outer = 0, total = 0, status = 2, fallbacks = 0, longest = 0;
     bool fp64 = false;
     const int max_outer = 60;
     double* r64 = ctx->d_t0;
     double* d64 = ctx->d_t1;
     PF_TRY(true_residual(ctx, b, x, r64, &rn));
     while (outer < max_outer) {
-        if (rn <= goal * bn) break;
+        const bool met = rn <= eps * bn;
+        if (rn <= goal * bn || (met && outer == 0)) break;
         if (total >= itrmax) break;
         PcgRun run;
         if (!fp64) {
+            const int cap = std::min(met ? longest : kInnerCap, itrmax - total);
             const double inner = parity ? std::max(0.125 * inner_eps, std::min(0.1, 0.1 * goal * bn / rn)) : inner_eps;
             k_convert<double, float><<<gsize(ctx->nv), kBlock, 0, ctx->stream>>>(ctx->nv, r64, ctx->f_b);
             PF_TRY(pcg_device<float>(ctx, false, ctx->f_b, ctx->f_x, ctx->f_D, ctx->f_r, ctx->f_z, ctx->f_p0,
-                                     ctx->f_p1, ctx->f_q, inner, std::min(kInnerCap, itrmax - total), run));
+                                     ctx->f_p1, ctx->f_q, inner, cap, run));
             total += run.iterations;
+            longest = std::max(longest, run.iterations);
             outer++;
             PF_HIP(hipMemcpyAsync(d64, x, sizeof(double) * ctx->nv, hipMemcpyDeviceToDevice, ctx->stream));
             k_axpy_f32<<<gsize(ctx->nv), kBlock, 0, ctx->stream>>>(ctx->nv, ctx->f_x, x);

@@ -115,6 +115,17 @@ def test_element_matrix_without_parity_blocks(pa):
     other.close()
 
 
+def test_mixed_solve_with_nothing_to_do(pa):
+    """x = 0 meets eps >= 1: no step is taken, resident or launched."""
+    ctx, b = problem(pa, 9, 5, 3)
+    for mode in (pa.PF_RESIDENT_AUTO, pa.PF_RESIDENT_OFF):
+        ctx.set_resident(mode)
+        for eps in (1.0, 3.0):
+            x, st = ctx.pcg(b, op=pa.PF_OP_EBE32, eps=eps)
+            assert (st["status"], st["iterations"], st["outer"]) == (1, 0, 0) and not np.any(x)
+    ctx.close()
+
+
 def test_default_operator_after_another(pa):
     """PF_H8_OP_AUTO brings a context back to the resident kernel, with the bits
     that it gave before."""
