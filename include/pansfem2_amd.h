@@ -189,8 +189,9 @@ int pf_pcg(pf_ctx* ctx, int op, const double* b_free, double* x_free, double eps
  * single-reduction forms follow Chronopoulos and Gear (p.Kp from u.Ku): one
  * reduction per iteration, the same iterates in exact arithmetic, the same
  * stopping test on the recursive residual, the Jacobi step as a product with
- * 1/D.  Grids whose vectors fit the registers and LDS of the chip (up to
- * about 650,000 nodes) are solved by one resident kernel in the first three
+ * 1/D.  Grids whose vectors fit the registers and LDS of the chip (256 compute
+ * units: up to 585,000 to 614,000 nodes by the grid's shape, 769 x 769 or
+ * 1086 x 543 elements) are solved by one resident kernel in the first three
  * forms; larger ones, and the recomputed form, launch every iteration:
  *   PF_PCG_SINGLE_REDUCTION_CARRIED: s = K p and w = K u carried as vectors
  *     (88 bytes per free DOF and iteration);
@@ -241,8 +242,8 @@ int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled);
  *   PF_H8_OP_MFMA: the element matrix as a batched product on the matrix
  *     cores (16 elements of one colour per product, K0 in registers), the
  *     rows summed per node in LDS in colour order (deterministic).
- *   PF_H8_OP_AUTO (the default): Jacobi-PCG solves of grids that fit the chip (up
- *     to about 128 x 64 x 64 elements) run in one resident kernel, with the
+ *   PF_H8_OP_AUTO (the default): Jacobi-PCG solves of grids that fit the chip (256
+ *     compute units: up to 128 x 64 x 64 elements) run in one resident kernel, with the
  *     element matrix in its parity basis where it has one (any box element of a
  *     material with the box's mirror planes), and the others use PF_H8_OP_VALU.
  * The other two are always launched.  Has no counterpart in the reference. */

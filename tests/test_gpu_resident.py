@@ -4,7 +4,9 @@ against the assembled-matrix solve, which launches every iteration.
 
 Grid shapes: one workgroup (with idle rows and lanes), a single row or column of
 elements, several workgroups with uneven tiles, every rows-per-thread variant,
-the largest grid that fits and the first that does not.  The first iterates
+the largest grids of some shapes that fit the chip and the next that do not; the
+context counts its resident solves, so that each test knows which kernel ran.
+The first iterates
 differ from the assembled solve's by the order of sums only: a few hundred
 roundings of 1e-16 per entry, 1e-12 with the head room of the recurrences.
 """
@@ -61,13 +63,19 @@ def test_iterates_against_assembled(pa, nx, ny, form):
     assert st["true_residual"] < 1e-7
     x2, _ = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-10)
     assert np.array_equal(x, x2)
+    assert ctx.resident_runs() == (5, 0)
     ctx.close()
 
 
-@pytest.mark.parametrize("nx,ny", [(1024, 512), (815, 791), (1023, 703)])
-def test_large_grids_against_recomputed_form(pa, nx, ny):
-    """Near the largest grid a chip holds, and one beyond it: the resident
-    forms against the launched recomputing form."""
+# square, 2:1, 3:2, 8:3 and 4:1 grids of 584,000 to 614,000 nodes that fit 256
+# workgroups of 150 KB LDS (12 x 8 bytes a node, its rows padded to five), the
+# next of some of these shapes, and larger ones
+@pytest.mark.parametrize("nx,ny,fits", [(1024, 512, True), (769, 769, True), (1086, 543, True), (958, 639, True),
+                                        (1279, 479, True), (1536, 384, True), (770, 770, False), (1088, 544, False),
+                                        (815, 791, False), (1023, 703, False)])
+def test_large_grids_against_recomputed_form(pa, nx, ny, fits):
+    """Near the largest grid a chip holds, and beyond it: the resident (or then
+    the launched) forms against the launched recomputing form."""
     print(f"resident large {nx}x{ny}", flush=True)
     ctx, b = problem(pa, nx, ny)
     xs = {}
@@ -77,6 +85,7 @@ def test_large_grids_against_recomputed_form(pa, nx, ny):
         assert st["iterations"] == 40 and st["status"] == 2
     for form in (0, 2):
         assert rel(xs[form], xs[3]) < 1e-11, rel(xs[form], xs[3])
+    assert ctx.resident_runs() == (2 if fits else 0, 0)
     ctx.close()
 
 
