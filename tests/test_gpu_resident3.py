@@ -2,8 +2,10 @@
 matrix in its parity basis, shared nodes' sums completed axis by axis) against
 the assembled-matrix solve, and the rule that decides on the parity basis.
 
-Shapes: one box, boxes of uneven sizes along every axis, one layer per half box
-and none, 16 elements along a box's edge.  The first iterates differ from the
+Shapes: one box, one layer per half box and none, 16 elements along a box's edge,
+boxes split along one, two and all three axes (nodes with two, four and eight
+holders) in equal and unequal parts, both sizes of the kernel (4 and 16 values
+per thread).  The first iterates differ from the
 assembled solve's by the order of sums and the transforms' roundings: some
 hundreds of 1e-16 per entry, 1e-12 with the head room of the recurrences.
 """
@@ -52,6 +54,58 @@ def test_iterates_against_assembled(pa, nx, ny, nz):
     x32, s32 = ctx.pcg(b, op=pa.PF_OP_EBE32, eps=1e-9)
     assert s32["status"] == 1 and s32["true_residual"] <= 1.0000001e-9
     assert rel(x32, xr) < 1e-6
+    assert ctx.resident_runs() == (5 + s32["outer"], 0)
+    ctx.close()
+
+
+# 256 workgroups: 30x4x2 boxes, 24x5x2 and 14x6x3 uneven ones (4 values per
+# thread); 15x5x3 uneven along j and k and 10x6x4 uneven along all axes (16)
+@pytest.mark.parametrize("nx,ny,nz", [(60, 30, 30), (47, 26, 23), (41, 33, 35), (75, 37, 39), (97, 47, 51)])
+def test_boxes_split_along_three_axes(pa, nx, ny, nz):
+    print(f"hex8 resident {nx}x{ny}x{nz}", flush=True)
+    ctx, b = problem(pa, nx, ny, nz)
+    ctx.assemble_csr()
+    for k in (1, 2, 6, 25):
+        xr, sr = ctx.pcg(b, op=pa.PF_OP_CSR64, eps=1e-30, itrmax=k)
+        x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-30, itrmax=k)
+        assert st["iterations"] == sr["iterations"] == k
+        assert rel(x, xr) < 1e-12, (k, rel(x, xr))
+    assert ctx.resident_runs() == (4, 0)
+    ctx.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz,fits", [(128, 64, 64, True), (132, 66, 66, False)])
+def test_largest_boxes_against_launched(pa, nx, ny, nz, fits):
+    """16x4x4 boxes of 8x16x16 elements, the largest that the kernel takes, with
+    random densities, and a grid beyond it."""
+    ctx, b = problem(pa, nx, ny, nz)
+    for k in (6, 25):
+        x, st = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-30, itrmax=k)
+        ctx.set_resident(pa.PF_RESIDENT_OFF)
+        xr, sr = ctx.pcg(b, op=pa.PF_OP_EBE64, eps=1e-30, itrmax=k)
+        ctx.set_resident(pa.PF_RESIDENT_AUTO)
+        assert st["iterations"] == sr["iterations"] == k and rel(x, xr) < 1e-12, (k, rel(x, xr))
+    assert ctx.resident_runs() == (2 if fits else 0, 0)
+    ctx.close()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(17, 9, 5), (47, 26, 23), (75, 37, 39)])
+def test_fp32_operator_by_the_work_it_takes(pa, nx, ny, nz):
+    """The refinement hides a wrong FP32 operator in the solution, not in the
+    steps and inner iterations it takes.  The resident solve aims at an eighth of
+    inner_eps and eps, and its operator's roundings are smaller: its steps are as
+    many or one fewer, its iterations fewer (602 and 833 in 3 and 3 steps, 1705
+    and 2021 in 3 and 3, 2721 and 4177 in 3 and 4); a quarter more than the
+    launched solve's is a wrong operator."""
+    ctx, b = problem(pa, nx, ny, nz)
+    x, st = ctx.pcg(b, op=pa.PF_OP_EBE32, eps=1e-9)
+    assert ctx.resident_runs()[0] == st["outer"]
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
+    xl, sl = ctx.pcg(b, op=pa.PF_OP_EBE32, eps=1e-9)
+    print(st, sl, flush=True)
+    assert st["status"] == sl["status"] == 1 and st["fallbacks"] == sl["fallbacks"] == 0
+    assert abs(st["outer"] - sl["outer"]) <= 1 and st["iterations"] <= 1.25 * sl["iterations"]
+    assert rel(x, xl) < 1e-6
     ctx.close()
 
 

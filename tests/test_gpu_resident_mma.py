@@ -1,12 +1,15 @@
 """GPU parity of the resident MMA / CONLIN update (k_mma_resident: one launch per
-update) against the oracle's UpdateVariables, at sizes around the borders of its
-variants: one workgroup with idle lanes, several, and one, two and four
-variables per thread (the borders are 131072 and 262144 variables on 256
-compute units).
+update) against the launched kernels, which the loops compare with the
+reference's, at sizes around the borders of its variants: one workgroup with
+idle lanes, several, and one, two and four variables per thread (the borders
+are 131072 and 262144 variables on 256 compute units, the end 524288), and,
+independently of both, against the solution of the subproblem.
 
-The sums over n variables are added in another order than the oracle's: about
-sqrt(n) 1e-16 of their magnitude, which the interior point (ended at 1e-7)
-passes on to x; 1e-9 holds with head room, as for the loops.
+The sums over n variables are added in another order: about sqrt(n) 1e-16 of
+their magnitude, which the interior point (ended at 1e-7) passes on to x; 1e-9
+holds with head room, as for the loops.  The asymptotes are formed variable by
+variable from x's history, with the same operations in both, so that they
+differ by what x differs.
 """
 import numpy as np
 import pytest
@@ -15,15 +18,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("kind", ["mma", "conlin"])
-@pytest.mark.parametrize("nx,ny", [(3, 1), (32, 16), (40, 13), (120, 40), (363, 361), (512, 257), (521, 511)])
-def test_updates_against_launched_arithmetic(nx, ny, kind):
+@pytest.mark.parametrize("nx,ny", [(3, 1), (32, 16), (40, 13), (120, 40), (363, 361), (512, 257), (521, 511),
+                                   (1024, 512), (1025, 512)])
+def test_updates_against_launched_and_solution(nx, ny, kind):
     import pansfem2_amd as pa
     print(f"resident {kind} {nx}x{ny}", flush=True)
     n = nx * ny
     rng = np.random.default_rng(n)
-    ctx = pa.cantilever2d(nx, ny)
-    (ctx.mma_init if kind == "mma" else ctx.conlin_init)()
-    update = ctx.mma_update if kind == "mma" else ctx.conlin_update
+    ctx, launched = pa.cantilever2d(nx, ny), pa.cantilever2d(nx, ny)
+    launched.set_resident(pa.PF_RESIDENT_OFF)
+    update, update2 = ((c.mma_update if kind == "mma" else c.conlin_update) for c in (ctx, launched))
+    for c in (ctx, launched):
+        (c.mma_init if kind == "mma" else c.conlin_init)()
     xs = rng.uniform(0.2, 0.8, n)
     prev = []
     for it in range(4):
@@ -32,9 +38,16 @@ def test_updates_against_launched_arithmetic(nx, ny, kind):
         g = float(xs.sum() / (0.5 * n) - 1.0)
         new, steps = update(xs, 1.0 + it, df, g, dg)
         assert 5 < steps < 200
+        # both contexts are given the same x, so that each update is compared by itself
+        new2, steps2 = update2(xs, 1.0 + it, df, g, dg)
+        assert steps == steps2
+        assert np.max(np.abs(new - new2)) < 1e-9, np.max(np.abs(new - new2))
         st = ctx.mma_get_state()
         assert st["k"] == it + 1 and np.array_equal(st["xkm1"], xs)
         assert it == 0 or np.array_equal(st["xkm2"], prev[-1])
+        if kind == "mma":
+            st2 = launched.mma_get_state()
+            assert np.array_equal(st["L"], st2["L"]) and np.array_equal(st["U"], st2["U"])
         ref = subproblem(kind, xs, prev, df, g, dg, st)
         # the interior point ends at eps = 1e-7: x is within its barrier's bias
         # of the subproblem's solution, the same at every size
@@ -42,6 +55,8 @@ def test_updates_against_launched_arithmetic(nx, ny, kind):
         assert np.all(new >= 0.01 - 1e-12) and np.all(new <= 1.0 + 1e-12)
         prev.append(xs)
         xs = new
+    assert ctx.resident_runs() == (4 if n <= 524288 else 0, 0) and launched.resident_runs() == (0, 0)
+    launched.close()
     # the same inputs give the same bits
     ctx2 = pa.cantilever2d(nx, ny)
     (ctx2.mma_init if kind == "mma" else ctx2.conlin_init)()

@@ -4,8 +4,10 @@ in numpy with the filter applied in every step: the same decisions, lambda and
 steps (the volumes differ by rounding, about 1e-15, and none of these decisions
 is that close), and x+ to the last bits of its formula.
 
-Sizes: one workgroup with idle lanes, several, the borders between one, two and
-four elements per thread, both element types, a radius that reaches past one ring.
+Sizes: one workgroup with idle lanes, several, the borders between one, two,
+four, eight and sixteen elements per thread (131072 times those on 256 compute
+units) and beyond the last, which is launched, both element types, a radius that
+reaches past one ring.
 """
 import numpy as np
 import pytest
@@ -13,8 +15,11 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("R", [1.5, 0.5, 2.3])
-@pytest.mark.parametrize("shape", [(1, 1), (7, 3), (120, 40), (37, 41), (363, 361), (512, 257), (5, 3, 4), (33, 17, 16)])
+SHAPES = [(1, 1), (7, 3), (120, 40), (37, 41), (363, 361), (512, 257), (5, 3, 4), (33, 17, 16)]
+LARGE = [(1024, 512), (1025, 512), (1024, 1025), (2048, 1024), (2049, 1024), (128, 90, 90)]
+
+
+@pytest.mark.parametrize("shape,R", [(s, R) for R in (1.5, 0.5, 2.3) for s in SHAPES] + [(s, 1.5) for s in LARGE])
 def test_bisection_against_numpy(shape, R):
     import pansfem2_amd as pa
     print(f"resident OC {shape} R {R}", flush=True)
@@ -37,6 +42,7 @@ def test_bisection_against_numpy(shape, R):
         new, lam_dev, steps_dev = ctx.oc_update(x, df, dg)
         assert lam_dev == lam and steps_dev == steps
         assert np.max(np.abs(new - ref)) < 1e-15
+    assert ctx.resident_runs() == (2 if n <= 16 * 131072 else 0, 0)
     # another radius: the column sums follow
     ctx.filter_setup(1.1)
     new, lam_dev, _ = ctx.oc_update(x, df, dg, lambdaeps=1e-2)
