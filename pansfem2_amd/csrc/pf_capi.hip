@@ -627,7 +627,10 @@ struct Res3Shape {
 // 1.5 per pass over a layer of each half box (two waves per SIMD from 9 element
 // rows on), 0.001 per node value, 1.8 per split axis (an exchange), 0.0008 per
 // exchanged face value.  60x30x30: 30x4x2 boxes 13.2, 15x4x4 15.0, 12x3x3 21.0;
-// 128x64x64: 16x4x4 31.6, 8x8x4 39 to 44.
+// 128x64x64: 16x4x4 31.6, 8x8x4 39 to 44.  Values per thread: 4 while they
+// suffice, else 16, the most that a box of 16 x 16 rows and 8 layers has; sizes
+// between (80x40x40 has 5, 100x40x40 6, 100x50x50 10) pay for 16: 25.5, 26.5 and
+// 31.6 us, launched 48.7, 48.7 and 55.8.
 template <class T>
 Res3Shape res3_pick(const pf_ctx* ctx) {
     Res3Shape best;
@@ -2194,7 +2197,9 @@ void net_input(pf_ctx* ctx, const double* rho, const double* r, double rs, const
 // Over the V-cycle the two pieces run side by side: its coarse levels occupy a
 // few of the CUs, the network's kernels the others.  They share no buffer that
 // either writes, and the caller's stream waits for both, so nothing changes but
-// the time: a learned solve at 1024 x 512 takes 15.3 ms, 17.5 one after the other.
+// the time: a learned solve at 1024 x 512 takes 14.1 ms, 16.5 one after the other,
+// in a process with one context; after other contexts' work, whose streams share
+// the process's four hardware queues with these two, 17.2 and 18.0.
 int net_parts(pf_ctx* ctx, const double* rho, const double* r, double rn, const double* rn_dev = nullptr) {
     LearnedNet* N = ctx->net;
     const long nv = ctx->nv;

@@ -326,7 +326,8 @@ __global__ void __launch_bounds__(256) k_conlin_trial(long n, double tau, double
 // ------------------------------------------------- resident update -----
 // The whole UpdateVariables in one cooperative launch: the approximation, the
 // interior point and the Newton direction of S variables per thread stay in
-// registers (17 values each), the scalar algebra runs in every thread on sums
+// registers (17 values each; with four variables 41 of them, CONLIN 25, go to
+// scratch), the scalar algebra runs in every thread on sums
 // that all workgroups add in one order (res_publish, res_collect).  The
 // launched form reads and writes 16 vectors per Newton step and returns to
 // the host four times for its sums.  Measured through pf_mma_update (host

@@ -21,13 +21,18 @@
 // a + b = b + a every holder of a node has the same bits.  Each global node is
 // counted and written by one holder.  p and q live in LDS, r and the diagonal in
 // registers; x is read and written once an iteration, in the order of the
-// workgroup's own values, through the L2 that holds it.
+// workgroup's own values, through the L2 that holds it.  FP64 with 16 values per
+// thread is the exception: beside the operator's four faces r, d and z do not
+// fit, 64 of its vector registers (244 bytes a lane) go to scratch, and all
+// variants keep about 200 scalars in lanes of vector registers.
 //
 // Measured per iteration (launched kernels before, resident now): 128x64x64
-// FP64 69 us, 32 us; 60x30x30 FP64 35, 13, FP32 28, 10; 16x8x8 31, 8.  Of the 32
-// us at 128x64x64 the operator takes 10 (its FP64 issue bounds it at 3.5; one or
-// two waves a SIMD leave the rest to latency), the three face exchanges 9, the
-// vector updates and their exchange 9.
+// FP64 68 us, 32 us; 100x50x50 56, 32; 100x40x40 49, 26; 80x40x40 49, 25;
+// 60x30x30 FP64 35, 13, FP32 28, 10; 16x8x8 31, 8.  Of the 32 us at 128x64x64 (by
+// the clock in workgroup 0) the operator takes 9.6 (its FP64 issue bounds it at
+// 3.5; one or two waves a SIMD leave the rest to latency), the three face
+// exchanges 9.5, p and p.Kp 1.8, the update of r and x and the new z 4.5, the two
+// sums' waits 5.8; of the 13.5 us at 60x30x30 3.2, 4.8, 0.6, 1.5 and 3.0.
 #pragma once
 
 namespace pf {
@@ -585,11 +590,14 @@ __global__ void __launch_bounds__(256) k_filter_colsum(G3 g, int dim, int win, d
 
 // The whole bisection of an OC update with the density filter (no projection) in
 // one cooperative launch: x, the derivatives and the filter's column sums of S
-// elements per thread stay in registers.  The filter is linear, so the filtered
-// volume is the column sums' product with x+, the same sum in another order, and
-// a step is S candidates and one exchanged sum.  The launched form filters x+
-// in every step: per step 8.6 us at 120x40 and 36 at 128x64x64; resident 2.3
-// and 2.1, bound by the exchange.
+// elements per thread stay in registers (of sixteen, 170 go to scratch).  The
+// filter is linear, so the filtered volume is the column sums' product with x+,
+// the same sum in another order, and a step is S candidates and one exchanged
+// sum, whose latency bounds it on small grids.  The launched form filters x+ in
+// every step.  A launch takes 72 us at 120x40 (2.3 per step; launched 8.6) and
+// 102 at 128x64x64 (launched 36 per step); a whole update with host vectors,
+// launched and resident: 120x40 0.38, 0.20 ms; 1024x512 (four per thread) 1.31,
+// 0.78; 1024x1000 (eight) 2.46, 1.50; 2048x1024 (sixteen) 5.32, 3.69.
 struct OcRes {
     long n;
     int max_steps;
