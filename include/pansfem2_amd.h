@@ -213,25 +213,38 @@ int pf_set_pcg_form(pf_ctx* ctx, int form);
 /* Jacobi-PCG solves with the matrix-free operators, MMA and CONLIN updates and
  * OC bisections without projection run in one resident kernel where the grid
  * fits the chip, and in kernels launched per iteration (per Newton or bisection
- * step) otherwise: on larger grids, where a cooperative launch is refused or
- * the resident kernel's buffers cannot be had, and after a stall (a resident
- * kernel's workgroups have waited two seconds for one another): the call then
- * starts over launched, and so does the next one run, after a second stall in
- * a row the next two, and so on up to 1024.  Until changed:
- *   PF_RESIDENT_AUTO: so (the default);
+ * step) otherwise: on larger grids, where the resident kernel's buffers cannot
+ * be had, and after
+ *   - a stall (a resident kernel's workgroups have waited two seconds for one
+ *     another): the call starts over launched, and so does the next one run,
+ *     after a second stall in a row the next two, and so on up to 1024;
+ *   - a refused cooperative launch (another process on the GPU has made one
+ *     and still runs): this call and the next 1024 are launched.
+ * The two sum in different orders, so that results agree to rounding and are
+ * the same bits from run to run only where the same kernels ran: beside other
+ * processes, with PF_RESIDENT_OFF.  Until changed:
+ *   PF_RESIDENT_AUTO: as above (the default);
  *   PF_RESIDENT_OFF: always launched;
  *   PF_RESIDENT_STALL: as AUTO, but a resident solve's launches (2048
  *     iterations each; an update or bisection is one launch) after the first
- *     `after` end as stalled, as beside a program that keeps the GPU busy;
+ *     `after` end as stalled;
  *   PF_RESIDENT_NOMEM: as AUTO, but of the buffers that resident kernels still
- *     have to allocate, those after the first `after` are not to be had.
- * The last two are for tests of what follows; the others do not use `after`.
+ *     have to allocate, those after the first `after` are not to be had;
+ *   PF_RESIDENT_REFUSED: as AUTO, but every cooperative launch is refused.
+ * The last three are for tests of what follows; `after` is not used otherwise.
  * Has no counterpart in the reference. */
-enum { PF_RESIDENT_AUTO = 0, PF_RESIDENT_OFF = 1, PF_RESIDENT_STALL = 2, PF_RESIDENT_NOMEM = 3 };
+enum {
+    PF_RESIDENT_AUTO = 0,
+    PF_RESIDENT_OFF = 1,
+    PF_RESIDENT_STALL = 2,
+    PF_RESIDENT_NOMEM = 3,
+    PF_RESIDENT_REFUSED = 4
+};
 int pf_set_resident(pf_ctx* ctx, int mode, int after);
 /* How many solves (inner solves of a mixed one each), updates and bisections
- * of this context have run resident to their end, and how many have stalled. */
-int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled);
+ * of this context have run resident to their end, and how many gave way by a
+ * stall or a refused launch. */
+int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* gave_way);
 /* Kernel of the hex8 matrix-free operator inside the fused PCG iteration
  * (pf_pcg, pf_pcg_dev, pf_simp_run and the multigrid PCG's outer FP64
  * operator on hex8 grids), until changed.  Both apply the same operator as

@@ -21,7 +21,7 @@ PF_PCG_SINGLE_REDUCTION_CARRIED, PF_PCG_SINGLE_REDUCTION_RECOMPUTED = 2, 3
 PF_MG_PROLONG_BILINEAR, PF_MG_PROLONG_STIFFNESS = 0, 1
 PF_MG_RESIDUAL_AUTO, PF_MG_RESIDUAL_NODE, PF_MG_RESIDUAL_ELEMENT = 0, 1, 2
 PF_H8_OP_AUTO, PF_H8_OP_VALU, PF_H8_OP_MFMA = -1, 0, 1
-PF_RESIDENT_AUTO, PF_RESIDENT_OFF, PF_RESIDENT_STALL, PF_RESIDENT_NOMEM = 0, 1, 2, 3
+PF_RESIDENT_AUTO, PF_RESIDENT_OFF, PF_RESIDENT_STALL, PF_RESIDENT_NOMEM, PF_RESIDENT_REFUSED = 0, 1, 2, 3, 4
 
 _i32p = np.ctypeslib.ndpointer(np.int32, flags="C_CONTIGUOUS")
 _f64p = np.ctypeslib.ndpointer(np.float64, flags="C_CONTIGUOUS")
@@ -359,12 +359,14 @@ class Context:
         CONLIN update and OC bisection where the grid fits the chip),
         PF_RESIDENT_OFF (always the launched kernels); for tests of the
         fallback PF_RESIDENT_STALL (resident launches after the first `after`
-        of a solve end as stalled) and PF_RESIDENT_NOMEM (the buffers they
-        allocate after the first `after` cannot be had)."""
+        of a solve end as stalled), PF_RESIDENT_NOMEM (the buffers they
+        allocate after the first `after` cannot be had) and
+        PF_RESIDENT_REFUSED (no cooperative launch is made)."""
         self._ck(lib().pf_set_resident(self._h, mode, after))
 
     def resident_runs(self):
-        """(ended, stalled): resident solves, updates and bisections so far."""
+        """(ended, gave way): resident solves, updates and bisections so far
+        that ran to their end, and that stalled or were refused."""
         d, s = ctypes.c_int64(0), ctypes.c_int64(0)
         self._ck(lib().pf_resident_runs(self._h, ctypes.byref(d), ctypes.byref(s)))
         return d.value, s.value

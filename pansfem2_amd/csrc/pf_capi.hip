@@ -259,7 +259,7 @@ void free_grid(pf_ctx* ctx) {
     dfree(ctx->res_halo);
     dfree(ctx->res_loc);
     ctx->res_halo_n = ctx->res_loc_n = 0;
-    ctx->res_pause = ctx->res_backoff = 0;
+    if (ctx->res_backoff) ctx->res_pause = ctx->res_backoff = 0;
     dfree(ctx->d_e0); dfree(ctx->d_e1); dfree(ctx->d_e2); dfree(ctx->d_e3); dfree(ctx->d_e4); dfree(ctx->d_e5);
     dfree(ctx->d_e6);
     dfree(ctx->d_cg); dfree(ctx->d_load);
@@ -498,12 +498,26 @@ bool res_gave_up(pf_ctx* ctx) {
     if (!ctx->h_res->stall) return false;
     ctx->res_backoff = std::min(1024, std::max(1, 2 * ctx->res_backoff));
     ctx->res_pause = ctx->res_backoff + 1;  // res_enter of the call that tries again takes the last one
-    ctx->res_stalls++;
+    ctx->res_gave++;
     return true;
 }
 void res_ended(pf_ctx* ctx) {
     ctx->res_backoff = 0;
     ctx->res_done++;
+}
+// A cooperative launch.  Refused (false), the next 1024 calls are launched: the
+// runtime takes 40 ms to refuse (a 16x8 solve takes 2 ms launched), and it does
+// so as long as another process that has made such a launch lives.
+bool res_launch(pf_ctx* ctx, const void* kern, unsigned wgs, int nt, void** args, size_t lds) {
+    if (ctx->res_mode != PF_RESIDENT_REFUSED) {
+        if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(nt), args, (unsigned)lds, ctx->stream) == hipSuccess)
+            return true;
+        (void)hipGetLastError();
+    }
+    ctx->res_backoff = 0;  // not a stall: a new grid does not end the pause
+    ctx->res_pause = 1024 + 1;
+    ctx->res_gave++;
+    return false;
 }
 
 constexpr int kResChunk = 2048;  // iterations per launch: other streams get the GPU in between
@@ -561,12 +575,7 @@ int res_run(pf_ctx* ctx, const void* kern, int wgs, int nt, size_t lds, ARGS& A,
         A.tag = ctx->res_tag;
         ctx->res_tag += 2 * (A.m1 - A.m0) + 2;
         void* args[] = {&A};
-        if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(nt), args, (unsigned)lds, ctx->stream) != hipSuccess) {
-            (void)hipGetLastError();
-            if (m == 0) return PF_OK;
-            ctx->err = "hipLaunchCooperativeKernel failed inside a resident solve";
-            return PF_ERR_HIP;
-        }
+        if (!res_launch(ctx, kern, wgs, nt, args, lds)) return PF_OK;
         PF_HIP(hipMemcpyAsync(ctx->h_pcg, A.S, sizeof(PcgDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
         PF_TRY(sync(ctx));
@@ -2787,10 +2796,7 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     res_force(ctx, 0);
     void* args[] = {&A};
     const unsigned wgs = (unsigned)((ne + (long)NT * S - 1) / ((long)NT * S));
-    if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(NT), args, 0, ctx->stream) != hipSuccess) {
-        (void)hipGetLastError();
-        return PF_OK;
-    }
+    if (!res_launch(ctx, kern, wgs, NT, args, 0)) return PF_OK;
     PF_HIP(hipMemcpyAsync(ctx->h_oc, ctx->d_oc, sizeof(OcDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_TRY(sync(ctx));
@@ -3009,10 +3015,7 @@ int mma_update_resident(pf_ctx* ctx, double* xk, const double* dfdx, double g, c
     res_force(ctx, 0);
     void* args[] = {&A};
     const unsigned wgs = (unsigned)((M->n + (long)NT * S - 1) / ((long)NT * S));
-    if (hipLaunchCooperativeKernel(kern, dim3(wgs), dim3(NT), args, 0, ctx->stream) != hipSuccess) {
-        (void)hipGetLastError();
-        return PF_OK;
-    }
+    if (!res_launch(ctx, kern, wgs, NT, args, 0)) return PF_OK;
     PF_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, sizeof(ResDev), hipMemcpyDeviceToHost, ctx->stream));
     PF_TRY(sync(ctx));
     if (res_gave_up(ctx)) return PF_OK;
@@ -3721,17 +3724,17 @@ int pf_set_pcg_form(pf_ctx* ctx, int form) {
 
 int pf_set_resident(pf_ctx* ctx, int mode, int after) {
     if (!ctx) return PF_ERR_ARG;
-    PF_CHECK(mode >= PF_RESIDENT_AUTO && mode <= PF_RESIDENT_NOMEM && after >= 0, PF_ERR_ARG,
+    PF_CHECK(mode >= PF_RESIDENT_AUTO && mode <= PF_RESIDENT_REFUSED && after >= 0, PF_ERR_ARG,
              "pf_set_resident: unknown mode");
     ctx->res_mode = mode;
     ctx->res_after = after;
     return PF_OK;
 }
 
-int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* stalled) {
+int pf_resident_runs(pf_ctx* ctx, int64_t* done, int64_t* gave_way) {
     if (!ctx) return PF_ERR_ARG;
     if (done) *done = ctx->res_done;
-    if (stalled) *stalled = ctx->res_stalls;
+    if (gave_way) *gave_way = ctx->res_gave;
     return PF_OK;
 }
 

@@ -133,9 +133,11 @@ struct pf_ctx {
     pf::ResDev *d_res = nullptr, *h_res = nullptr;
     unsigned res_tag = 1;
     int res_wgs = 0;
-    int res_pause = 0, res_backoff = 0;  // calls still to be launched after a stall (res_gave_up)
+    // calls still to be launched after a stall or a refused launch, and the last
+    // stall's number of them (res_gave_up, res_launch)
+    int res_pause = 0, res_backoff = 0;
     int res_mode = PF_RESIDENT_AUTO, res_after = 0;  // pf_set_resident
-    int64_t res_done = 0, res_stalls = 0;            // pf_resident_runs
+    int64_t res_done = 0, res_gave = 0;              // pf_resident_runs
 
     // MMA state
     struct MmaState* mma = nullptr;

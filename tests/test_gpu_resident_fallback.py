@@ -135,14 +135,12 @@ def test_stalled_mma_update(pa, n, kind):
         assert np.array_equal(a[i], b[i])
 
 
-@pytest.mark.parametrize("after", [0, 1])
-@pytest.mark.parametrize("dims,op", [((120, 40), "EBE64"), ((120, 40), "EBE32"), ((33, 16, 16), "EBE64"),
-                                     ((33, 16, 16), "EBE32")])
+@pytest.mark.parametrize("dims,op,after", [((120, 40), "EBE64", 0), ((120, 40), "EBE32", 0),
+                                           ((33, 16, 16), "EBE64", 0), ((33, 16, 16), "EBE64", 1),
+                                           ((33, 16, 16), "EBE32", 0), ((33, 16, 16), "EBE32", 1)])
 def test_solve_without_memory_for_the_exchange(pa, dims, op, after):
     """Resident solves allocate an exchange buffer, on hex8 another for x: where
     one of them cannot be had the launched kernels solve, which need neither."""
-    if after and len(dims) == 2:
-        pytest.skip("one buffer")
     ctx, b = problem(pa, dims)
     op = getattr(pa, "PF_OP_" + op)
     ctx.set_resident(pa.PF_RESIDENT_OFF)
@@ -176,9 +174,48 @@ def test_oc_update_without_memory_for_the_column_sums(pa):
     ctx.close()
 
 
+def test_refused_launches(pa):
+    """A refusal costs the runtime 40 ms, more than a small solve: it is asked
+    again after 1024 launched calls, also on a new grid, and every kind of call
+    gives the bits of the launched kernels meanwhile."""
+    ctx, b = problem(pa, (40, 13))
+    rng = np.random.default_rng(3)
+    x, df, dg = rng.uniform(0.2, 0.8, ctx.ne), -rng.uniform(0.05, 2.0, ctx.ne), np.full(ctx.ne, 1.0 / ctx.ne)
+
+    def calls():
+        ctx.mma_init()
+        return (ctx.pcg(b, eps=1e-8)[0], ctx.oc_update(x, df, dg)[0], ctx.mma_update(x, 1.0, df, 0.1, dg)[0],
+                ctx.pcg(b, op=pa.PF_OP_EBE32, eps=1e-8)[0])
+    ctx.set_resident(pa.PF_RESIDENT_OFF)
+    ref = calls()
+    for turn in range(4):  # each kind of call is the one refused
+        ctx.close()
+        ctx, b = problem(pa, (40, 13))
+        ctx.set_resident(pa.PF_RESIDENT_OFF)
+        ctx.mma_init()
+        first = (lambda: ctx.pcg(b, eps=1e-8), lambda: ctx.oc_update(x, df, dg),
+                 lambda: ctx.mma_update(x, 1.0, df, 0.1, dg), lambda: ctx.pcg(b, op=pa.PF_OP_EBE32, eps=1e-8))[turn]
+        want = first()
+        ctx.mma_init()
+        ctx.set_resident(pa.PF_RESIDENT_REFUSED)
+        got = first()
+        assert np.array_equal(got[0], want[0]) and ctx.resident_runs() == (0, 1)
+        for got, want in zip(calls(), ref):
+            assert np.array_equal(got, want)
+        assert ctx.resident_runs() == (0, 1)
+    ctx, b = problem(pa, (8, 4), ctx)
+    for _ in range(1025 - 4 - 1):
+        ctx.pcg(b, eps=1e-2)
+    assert ctx.resident_runs() == (0, 1)
+    ctx.set_resident(pa.PF_RESIDENT_AUTO)
+    ctx.pcg(b, eps=1e-2)
+    assert ctx.resident_runs() == (1, 1)
+    ctx.close()
+
+
 def test_mode_argument_checked(pa):
     ctx = pa.cantilever2d(8, 4)
-    for mode, after in ((4, 0), (-1, 0), (2, -1)):
+    for mode, after in ((5, 0), (-1, 0), (2, -1)):
         with pytest.raises(pa.PfError):
             ctx.set_resident(mode, after)
     ctx.close()
