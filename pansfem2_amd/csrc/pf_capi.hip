@@ -623,8 +623,9 @@ int pcg_resident(pf_ctx* ctx, bool sr, const T* b, T* x, const T* D, T* r, T* s,
     A.x = x; A.r = r; A.s = s; A.p = p; A.w = w;
     A.halo = ctx->res_halo;
     A.eps = eps;
+    const long end = std::max(itrmax, 0);  // pf_simp_run takes any cg_itrmax; the tags must go up
     // sr: step m finishes iterate m
-    return res_run(ctx, kern, sh.gi * sh.gj, sh.nt, sh.lds, A, sr ? (long)itrmax + 1 : itrmax, out, ran);
+    return res_run(ctx, kern, sh.gi * sh.gj, sh.nt, sh.lds, A, sr ? end + 1 : end, out, ran);
 }
 
 // Boxes of a hex8 resident solve.  gi == 0: the grid does not fit.
@@ -710,7 +711,7 @@ int pcg_resident3(pf_ctx* ctx, const T* b, T* x, const T* D, T* r, T* p, double 
     A.edge = ctx->res_halo;
     A.loc = (T*)ctx->res_loc;
     A.eps = eps;
-    return res_run(ctx, kern, wgs, kRes3Threads, sh.lds, A, itrmax, out, ran);
+    return res_run(ctx, kern, wgs, kRes3Threads, sh.lds, A, std::max(itrmax, 0), out, ran);
 }
 
 // Workgroups of k_cg1_q4_tile: full tiles, then edge tiles (launched first).

@@ -123,6 +123,26 @@ def test_more_iterations_than_one_launch(pa):
     ctx.close()
 
 
+def test_no_iterations_allowed(pa):
+    """itrmax = 0 gives x = 0, and so do the solves of a loop whose cg_itrmax is
+    negative (which the loop takes); the solves that follow do not see their
+    exchanges as their own (the tags go up all the same)."""
+    ctx, b = problem(pa, 17, 9, 5)
+    rho = np.full(ctx.ne, 0.5)
+    ctx.set_density(rho)
+    x, st = ctx.pcg(b, eps=1e-10)
+    x0, s0 = ctx.pcg(b, eps=1e-10, itrmax=0)
+    assert s0["status"] == 2 and s0["iterations"] == 0 and not np.any(x0)
+    for itrmax in (-1, -7, -1000, -2**31):
+        r = ctx.simp_run(1, pa.simp_default_params(cg_itrmax=itrmax))
+        assert r["status"] == pa.PF_NOT_CONVERGED and r["cg_iters"][0] == 0 and r["f"][0] == 0.0
+        ctx.set_density(rho)
+        x1, s1 = ctx.pcg(b, eps=1e-10)
+        assert s1["iterations"] == st["iterations"] and np.array_equal(x1, x)
+    assert ctx.resident_runs()[0] >= 10 and ctx.resident_runs()[1] == 0
+    ctx.close()
+
+
 def test_solve_that_ends_with_a_launch(pa):
     """A solve whose last iterate is the last of its first launch (2048): the
     second launch finds it converged before its first exchange, so that every
