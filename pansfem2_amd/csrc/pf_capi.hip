@@ -540,18 +540,23 @@ bool res_alloc(pf_ctx* ctx, T** p, long n, long* have) {
     return true;
 }
 
+// Before a launch, none of whose words are read by the next one: no word may
+// carry a tag that is still to come (a launch takes at most 5.2 million tags).
+void res_tags(pf_ctx* ctx) {
+    if (ctx->res_tag <= 0xf0000000u) return;
+    k_fill<u64><<<gsize(ctx->res_halo_n), kBlock, 0, ctx->stream>>>(ctx->res_halo_n, ctx->res_halo, 0ull);
+    k_fill<u64><<<1, kBlock, 0, ctx->stream>>>(2L * 4 * kResMaxWg * 2, ctx->res_slots, 0ull);
+    ctx->res_tag = 1;
+}
+
 // Exchange buffer of `words` words for a solve that starts now, and the
 // solve's scalars; *ok false: it cannot be had.
 int res_begin(pf_ctx* ctx, long words, bool* ok) {
     const bool fresh = ctx->res_halo_n < words;
     *ok = res_alloc(ctx, &ctx->res_halo, words, &ctx->res_halo_n);
     if (!*ok) return PF_OK;
-    if (fresh || ctx->res_tag > 0xf0000000u) {
-        // no word may carry a tag that is still to come
-        k_fill<u64><<<gsize(words), kBlock, 0, ctx->stream>>>(ctx->res_halo_n, ctx->res_halo, 0ull);
-        k_fill<u64><<<1, kBlock, 0, ctx->stream>>>(2L * 4 * kResMaxWg * 2, ctx->res_slots, 0ull);
-        ctx->res_tag = 1;
-    }
+    if (fresh) ctx->res_tag = 0xffffffffu;  // whatever the new words hold
+    res_tags(ctx);
     k_res_start<<<1, 1, 0, ctx->stream>>>((PcgDev*)ctx->d_pcg, ctx->d_res);
     return check_launch(ctx);
 }
@@ -568,6 +573,7 @@ int res_run(pf_ctx* ctx, const void* kern, int wgs, int nt, size_t lds, ARGS& A,
     const PcgDev* H = (const PcgDev*)ctx->h_pcg;
     int launch = 0;
     for (long m = 0;;) {
+        res_tags(ctx);
         res_force(ctx, launch++);
         A.m0 = (int)m;
         A.m1 = (int)std::min(end, m + kResChunk);
