@@ -2760,8 +2760,8 @@ int solve_nodal(pf_ctx* ctx, int op, const double* b, double* x, double eps, int
 
 // ------------------------------------------------------------------ OC ----
 // The bisection in one resident launch (k_oc_resident), its result in h_oc;
-// *ran is false, and nothing has been done, with the projection in the closure,
-// more elements than the chip's registers hold, no memory for the column sums or
+// *ran is false, and nothing has been done, with the projection in the closure, a
+// volume that is not a number, more elements than the chip's registers hold, no memory for the column sums or
 // a launch that cannot be made or stalled.
 int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const double* x, const double* dfdx,
                 const double* dgdx, double* xplus, bool* ran) {
@@ -2769,6 +2769,9 @@ int oc_resident(pf_ctx* ctx, const pf_oc_params* prm, int max_steps, const doubl
     constexpr int NT = kOcResThreads;
     const long ne = ctx->ne, most = (long)ctx->res_wgs * NT;
     if (!res_on(ctx) || ne > 16 * most || prm->beta > 0.0 || max_steps > 1000000) return PF_OK;
+    // a volume that divides by zero or scales by infinity is NaN where a term is
+    // zero: a single density's here, a whole neighbourhood's in the launched form
+    if (!(std::fabs(prm->vf * (double)ne) > 0.0) || !std::isfinite(prm->scale1)) return PF_OK;
     if (!ctx->have_fcol) {
         if (!res_alloc(ctx, &ctx->d_fcol, ne, &ctx->fcol_n)) return PF_OK;
         k_filter_colsum<<<gsize(ne), kBlock, 0, ctx->stream>>>(g3(ctx), ctx->dim, ctx->win, ctx->R, ctx->d_cg, nullptr,

@@ -50,3 +50,22 @@ def test_bisection_against_numpy(shape, R):
     assert np.array_equal(new, ctx2.oc_update(x, df, dg, lambdaeps=1e-2)[0])
     ctx.close()
     ctx2.close()
+
+
+@pytest.mark.parametrize("kw", [dict(vf=0.0), dict(vf=-0.0), dict(vf=float("nan")), dict(scale1=float("inf")),
+                                dict(vf=float("inf")), dict(scale1=0.0), dict(vf=-1.0), dict(lambdamin=0.0, lambdamax=0.0)])
+def test_unusual_volumes_as_launched(kw):
+    """Constraints that divide by zero, are infinite or say nothing, on a design
+    with single zero densities: decisions, lambda and x+ as launched."""
+    import pansfem2_amd as pa
+    ctx = pa.cantilever2d(40, 13)
+    rng = np.random.default_rng(1)
+    x, df, dg = rng.uniform(0.2, 0.8, ctx.ne), -rng.uniform(0.05, 2.0, ctx.ne), np.full(ctx.ne, 1.0 / ctx.ne)
+    x[::17] = 0.0
+    out = []
+    for mode in (pa.PF_RESIDENT_OFF, pa.PF_RESIDENT_AUTO):
+        ctx.set_resident(mode)
+        out.append(ctx.oc_update(x, df, dg, **kw) + (ctx.last_status,))
+    assert out[0][1:] == out[1][1:], (out[0][1:], out[1][1:])
+    assert np.array_equal(out[0][0], out[1][0])
+    ctx.close()
