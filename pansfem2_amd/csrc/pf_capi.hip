@@ -530,7 +530,10 @@ bool res_alloc(pf_ctx* ctx, T** p, long n, long* have) {
     if (*have >= n) return true;
     dfree(*p);
     *have = 0;
-    if (ctx->res_mode == PF_RESIDENT_NOMEM && ctx->res_after-- <= 0) return false;
+    if (ctx->res_mode == PF_RESIDENT_NOMEM) {
+        if (ctx->res_after <= 0) return false;
+        ctx->res_after--;
+    }
     if (hipMalloc((void**)p, sizeof(T) * (size_t)n) != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;
